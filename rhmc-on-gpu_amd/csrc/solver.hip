@@ -2955,6 +2955,10 @@ static int ms_cg_basis_group(std::vector<Context *> &cs, std::vector<GroupJob> &
     nmin = std::min(nmin, j.nrhs);
     cap_max = std::max(cap_max, br.cap);
   }
+  // the shape candidates run iteration 1 and read the iteration counter: on a
+  // fresh lead context it still holds 0, for which the operands would be the
+  // basis slot before the first
+  hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, c0.stream, iterc, 1);
   const int code = group_shape<R, LINK>(cs, runs, nmin);
   if (code < 0) return -1;
   // argument tables of the kChunk steps: [q][hop, M^dag M][lattice]

@@ -332,6 +332,37 @@ def test_c4b_six_uneven_lattices_in_lockstep(precision):
         g.close()
 
 
+def test_lockstep_first_on_fresh_handles():
+    """Handles whose first solve ever is a lockstep one (the launch shapes of
+    the group are timed before any lattice has iterated alone) give each
+    lattice the trajectory it runs alone on another handle: Delta H to 1e-9,
+    links to 1e-10 (FP64 solves)."""
+    lats = [(8, 8, 8, 4), (6, 4, 4, 6), (16, 8, 8, 8)]
+    first, md, last = rhmc_approximations(2, 1, 12, 8, 12)
+    co = dict(first=(first.a0, first.a, first.b), md=(md.a0, md.a, md.b), last=(last.a0, last.a, last.b))
+
+    def handles():
+        out = []
+        for i, d in enumerate(lats):
+            g = Gpu(d, mass=0.05, beta=5.6, n_pf=1, max_order=12)
+            g.init0(fields.random_links(fields.Lattice(*d), 70 + i, 0.3))
+            out.append(g)
+        return out
+
+    kws = [dict(n_flavours=2, no_md=2, integrator="omelyan", res_md=1e-10, res_metro=1e-10, relative=True,
+                bounds=(0.02, 5.6), draw_fields=True, seed=50 + i, **co) for i in range(len(lats))]
+    together, single = handles(), handles()
+    say("lockstep on fresh handles", lats)
+    res, st = multi_trajectory(together, kws)
+    assert st == [0] * len(lats)
+    for g, s, r, kw in zip(together, single, res, kws):
+        ra = s.trajectory(**kw)
+        assert abs(r.delta_h - ra.delta_h) < 1e-9
+        assert rel(g.end(ipdot=False, momenta=False)[0], s.end(ipdot=False, momenta=False)[0]) < 1e-10
+        g.close()
+        s.close()
+
+
 # ------------------------------------------------------------------ C5
 def test_c5_48c12_trajectory_delta_h():
     """C5: 48^3x12, Nf=2, am=0.01, beta=5.6, 2 pseudofermions, Omelyan 20
