@@ -25,10 +25,12 @@
 
 #include <algorithm>
 #include <cmath>
+#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -48,6 +50,7 @@ enum Slot {
   S_PARTIAL2, S_BASIS, S_BSH, S_HIST, S_COEF, S_HPART,
   S_FORCE_H, S_FORCE_COEF, S_SOLSUM_COEF,
   S_RS_SRC, S_RS_Y, S_RS_IDX, S_GROUP_TAB,
+  S_RES_H, S_RES_PART,
   S_COUNT
 };
 
@@ -77,6 +80,8 @@ struct Workspace {
   std::vector<DsArgs> group_tab;               // argument tables of the group's chunk (host copy)
   std::map<unsigned long long, int> group_tuned;  // lockstep launch shape per group composition
   long basis_kmax[2] = {0, 0};                 // most basis iterations a FP32 / FP64 solve needed
+  int num_cu = 0;                              // compute units of the device
+  bool resident_off = false;                   // a one-launch solve gave up waiting (device shared): not used again
   void *buf[S_COUNT] = {};
   size_t cap[S_COUNT] = {};
   unsigned *counter = nullptr;
@@ -101,6 +106,7 @@ Workspace *workspace_create(Context &c) {
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, c.device) == hipSuccess) {
     w->arch = prop.gcnArchName;
+    w->num_cu = prop.multiProcessorCount;
     const size_t colon = w->arch.find(':');
     if (colon != std::string::npos) w->arch.resize(colon);
   }
@@ -1268,6 +1274,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(ds_waves
   ds_ls_body<R, LINK, NR, MODE, RED>(a, blockIdx.x, gridDim.x);
 }
 
+}  // namespace rhmc
+#include "resident.hpp"
+namespace rhmc {
+
 // ---- several lattices in one launch.  The grid is the concatenation of
 // every lattice's own grid, each padded to a multiple of 8 workgroups so that
 // a lattice's local workgroup index keeps the XCD mapping of xcd_split
@@ -2362,6 +2372,7 @@ constexpr long kMaxSlots = 16384;
 constexpr size_t kMaxBasisBytes = 32ull << 30;
 constexpr int kBasisFull = 100;     // not even kMinBasis slots fit: the explicit-shift solver runs
 constexpr int kBasisRestart = 101;  // the basis filled: x holds the solutions so far (see BasisRestart)
+constexpr int kResidentGaveUp = 102;  // the one-launch iterations ran out of their wait (resident.hpp)
 constexpr long kMinBasis = 16;
 
 // Systems still running when the basis filled.  Their shifted residuals
@@ -2408,6 +2419,7 @@ struct BasisRun {
   DsArgs hop = {}, mdm = {};
   unsigned nbr = 0;
   bool timed = false;
+  bool resident = false;  // the iterations run as one launch
 };
 
 // buffers, scalar state and the first launches; the iteration counter
@@ -2718,6 +2730,9 @@ static int bms_finish(Context &c, BasisRun &br, double2 *x, int *iters_out, floa
   // the systems' final state (after the assembly: one wait for both)
   std::vector<MsState> &hs = br.hs;
   if (!d2h_sync(c, hs.data(), br.ms, sizeof(MsState) * nrhs)) return -1;
+  if (br.resident)
+    for (const MsState &q : hs)
+      if (q.nonfinite == kResAborted) return kResidentGaveUp;
   if (rs) {
     rs->res.resize(nrhs);
     rs->bnorm2.resize(nrhs);
@@ -2771,6 +2786,210 @@ static int bms_finish(Context &c, BasisRun &br, double2 *x, int *iters_out, floa
   return 0;
 }
 
+// Workgroups of the one-launch solves in flight on a device, as a share of
+// its compute units: solves of several handles (threads) run at the same
+// time only while all their workgroups fit, at most one per CU, so that
+// every grid is resident as a whole.
+class ResidentShare {
+ public:
+  ResidentShare(int device, double share) : d_(device < 0 || device >= kDevices ? 0 : device), s_(share) {
+    Slots &t = slots();
+    std::unique_lock<std::mutex> l(t.m);
+    t.cv.wait(l, [&] { return t.used[d_] + s_ <= 1.0 + 1e-9; });
+    t.used[d_] += s_;
+  }
+  ~ResidentShare() {
+    Slots &t = slots();
+    {
+      std::lock_guard<std::mutex> l(t.m);
+      t.used[d_] -= s_;
+    }
+    t.cv.notify_all();
+  }
+  ResidentShare(const ResidentShare &) = delete;
+  ResidentShare &operator=(const ResidentShare &) = delete;
+
+ private:
+  static constexpr int kDevices = 64;
+  struct Slots {
+    std::mutex m;
+    std::condition_variable cv;
+    double used[kDevices] = {};
+  };
+  static Slots &slots() {
+    static Slots t;
+    return t;
+  }
+  int d_;
+  double s_;
+};
+
+// One launch of k_bms_resident: the lattices of a solve that share it
+// (indices), the right-hand sides per member, threads per workgroup, each
+// lattice's sites per lane and workgroups per member.
+struct ResidentLaunch {
+  int nr = 1, threads = 512, sites_max = 1;
+  std::vector<int> lat, sites, nwg;
+  unsigned total = 0;  // workgroups
+};
+
+template <typename R, int LINK, int NR, int P>
+static int resident_per_cu(int threads) {
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_bms_resident<R, LINK, NR, P>, threads, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    n = 0;
+  }
+  return n;
+}
+// workgroups of a lattice's member, rounded up to the 8 XCDs
+static unsigned resident_wgs(const Context &c, int threads, int sites, int &nwg) {
+  const long per = (long)(threads / 4) * sites;
+  nwg = (int)((c.Vh + per - 1) / per);
+  return (unsigned)((nwg + 7) / 8 * 8);
+}
+
+// The launches of a solve over one or several lattices; empty where the
+// launches per iteration are used.  Measured per iteration (us, one launch
+// against the two tuned launches; FP64, FP32):
+//   8^3x4 1 to 8 systems  7.9 / 18,     7.5 / 18
+//   12^4  1               8.0 / 18,     7.0 / 17
+//   12^4  8 (4 a member) 19.9 / 28,    14.2 / 20
+//   16^4  1              12.0 / 22,     9.3 / 16
+//   16^4  2 (2 a member) 16.8 / 25,    12.5 / 18
+//   16^4  4 (4 a member) 25.4 / 28,    17.5 / 28
+//   16^4  8 (8 a member) 46   / 43,    32   / 28   (not taken)
+//   24^3x8 1 (two sites) 24.8 / 28,    17.7 / 19
+// The rule: the fewest systems per member (1, 2 or 4), then the smaller
+// workgroups, for which there is at most one workgroup per CU (16^4 with one
+// system: 14.5 us with 512 workgroups of 256 lanes).  One system on a lattice
+// too large for that may take two sites per lane (two systems of 16^4 that
+// way: 26 us).  Several lattices that do not fit that way
+// share the CUs as far as registers allow (the largest with two sites per
+// lane), else they run as up to three launches.
+template <typename R, int LINK>
+static std::vector<ResidentLaunch> resident_plan(const std::vector<Context *> &cs, const std::vector<BasisRun> &runs) {
+  const Workspace &w = *cs[0]->ws;
+  const int n = (int)cs.size();
+  if (w.resident_off || w.num_cu < 8 || getenv("RHMC_DSLASH_NR")) return {};
+  const unsigned cus = (unsigned)w.num_cu;
+  int nvec = 0;
+  bool split = true;  // every right-hand side's vectors are whole cache lines
+  for (int l = 0; l < n; l++) {
+    const size_t vb = (size_t)3 * cs[l]->Vh * sizeof(Cx<R>);
+    if (runs[l].timed || runs[l].nrhs * vb % 128) return {};
+    if ((size_t)cs[l]->Vh * 8 * sizeof(LinkRaw<R, LINK>) >= (1ull << 32)) return {};
+    nvec = std::max(nvec, runs[l].nrhs);
+    split = split && vb % 128 == 0;
+  }
+  auto all = [&](int nr, int threads, int sites) {
+    ResidentLaunch r;
+    r.nr = nr;
+    r.threads = threads;
+    r.sites_max = sites;
+    r.sites.assign(n, sites);
+    r.nwg.resize(n);
+    int members = 0;
+    for (int l = 0; l < n; l++) {
+      const int m = (runs[l].nrhs + nr - 1) / nr;
+      members += m;
+      r.lat.push_back(l);
+      r.total += resident_wgs(*cs[l], threads, sites, r.nwg[l]) * m;
+    }
+    if (members > kResMaxMembers || (!split && nr < nvec)) r.total = ~0u;
+    return r;
+  };
+  for (int nr = 1; nr <= 4; nr *= 2)
+    for (int threads = 256; threads <= 512; threads *= 2)
+      if (const ResidentLaunch r = all(nr, threads, 1); r.total <= cus) return {r};
+  if (n == 1) {
+    if (nvec == 1)
+      if (const ResidentLaunch r = all(1, 512, 2); r.total <= cus) return {r};
+    return {};
+  }
+  // several lattices, one system per member: as many workgroups as the CUs
+  // hold, the largest lattices with two sites per lane until they fit
+  ResidentLaunch r = all(1, 512, 1);
+  if (r.total != ~0u) {
+    const unsigned room = cus * (unsigned)resident_per_cu<R, LINK, 1, 2>(512);
+    r.sites_max = 2;
+    while (r.total > room) {
+      int big = -1;
+      for (int l = 0; l < n; l++)
+        if (r.sites[l] == 1 && (big < 0 || cs[l]->Vh > cs[big]->Vh)) big = l;
+      if (big < 0) break;
+      r.total -= (unsigned)((r.nwg[big] + 7) / 8 * 8) * runs[big].nrhs;
+      r.sites[big] = 2;
+      r.total += resident_wgs(*cs[big], 512, 2, r.nwg[big]) * runs[big].nrhs;
+    }
+    if (r.total <= room) return {r};
+  }
+  // in turn: the largest first, each into the first launch with room for it
+  std::vector<int> order(n);
+  for (int l = 0; l < n; l++) order[l] = l;
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cs[a]->Vh > cs[b]->Vh; });
+  std::vector<ResidentLaunch> out;
+  for (const int l : order) {
+    int nwg = 0;
+    const unsigned t = resident_wgs(*cs[l], 512, 1, nwg) * (unsigned)runs[l].nrhs;
+    if (t > cus || !split) return {};
+    size_t q = 0;
+    while (q < out.size() && out[q].total + t > cus) q++;
+    if (q == out.size()) out.emplace_back();
+    out[q].lat.push_back(l);
+    out[q].sites.push_back(1);
+    out[q].nwg.push_back(nwg);
+    out[q].total += t;
+  }
+  return out.size() <= 3 ? out : std::vector<ResidentLaunch>();
+}
+
+// all iterations of the launch's lattices on the first context's stream
+template <typename R, int LINK>
+static int resident_launch(const std::vector<Context *> &cs, std::vector<BasisRun> &runs, const ResidentLaunch &rl) {
+  Context &c0 = *cs[0];
+  ResGroup g = {};
+  const char *wait = getenv("RHMC_RESIDENT_WAIT");  // bound of a wait, 100 MHz ticks
+  g.wait = wait ? atoll(wait) : kResWaitTicks;
+  for (size_t q = 0; q < rl.lat.size(); q++) {
+    Context &c = *cs[rl.lat[q]];
+    BasisRun &br = runs[rl.lat[q]];
+    const long v = 3 * c.Vh;
+    Cx<R> *h = (Cx<R> *)ws_get(c, S_RES_H, sizeof(Cx<R>) * (size_t)(v * br.nrhs) * br.cap);
+    const int per = kResRing * kResCopies * res_copy(rl.nwg[q]), np = per * br.nrhs;
+    unsigned long long *part = (unsigned long long *)ws_get(c, S_RES_PART, sizeof(unsigned long long) * np + 64);
+    if (!h || !part) return -1;
+    hipLaunchKernelGGL(k_res_init, dim3(std::min(256, (np + kBlock - 1) / kBlock)), dim3(kBlock), 0, c0.stream, part,
+                       np, (int *)(part + np));
+    br.resident = true;
+    for (int r0 = 0; r0 < br.nrhs; r0 += rl.nr) {
+      ResArgs &a = g.a[g.n];
+      a.L = c.L;
+      a.U = link_ptr<LINK>(c);
+      a.basis = (Cx<R> *)br.basis + r0 * v;
+      a.h = h + r0 * v;
+      a.stride = v * br.nrhs;
+      a.nvec = std::min(rl.nr, br.nrhs - r0); a.nshift = br.nshift; a.cap = (int)br.cap;
+      a.part = part + (size_t)per * r0;
+      a.abort = (int *)(part + np);
+      a.diag = c.mass * c.mass;
+      a.sh = br.bsh + r0; a.ms = br.ms + r0; a.hist = br.hist + (size_t)r0 * br.cap * br.nshift;
+      a.nwg = rl.nwg[q];
+      a.sites = rl.sites[q];
+      g.start[g.n + 1] = g.start[g.n] + (unsigned)((a.nwg + 7) / 8 * 8);
+      g.n++;
+    }
+  }
+  const dim3 grid(g.start[g.n]), block((unsigned)rl.threads);
+#define RES_RUN(NR, P) hipLaunchKernelGGL((k_bms_resident<R, LINK, NR, P>), grid, block, 0, c0.stream, g)
+  if (rl.nr == 1 && rl.sites_max == 1) RES_RUN(1, 1);
+  else if (rl.nr == 1) RES_RUN(1, 2);
+  else if (rl.nr == 2) RES_RUN(2, 1);
+  else RES_RUN(4, 1);
+#undef RES_RUN
+  return hip_ok(c0, hipGetLastError(), "one-launch solve") ? 0 : -1;
+}
+
 // multi-shift CG with the stored residual basis on one lattice; x (FP64)
 // receives [nrhs][nshift] solutions (or x32 in FP32).  Returns kBasisFull
 // when not even kMinBasis slots fit (the caller then runs the
@@ -2780,10 +2999,25 @@ template <typename R, int LINK>
 static int ms_cg_basis(Context &c, const double2 *b, int nrhs, int nshift, const double *shifts,
                        const double *res_abs, int max_iter, double2 *x, int *iters_out, float2 *x32,
                        bool asm_fp32, BasisRestart *rs, double tol_abs = 0.0, double tol_rel = 0.0) {
-  BasisRun br;
+  std::vector<BasisRun> runs(1);
+  BasisRun &br = runs[0];
   int *iterc = iter_ptr(c);
-  const int rc = bms_setup<R, LINK>(c, br, b, nrhs, nshift, shifts, res_abs, max_iter, iterc, tol_abs, tol_rel);
+  int rc = bms_setup<R, LINK>(c, br, b, nrhs, nshift, shifts, res_abs, max_iter, iterc, tol_abs, tol_rel);
   if (rc) return rc;
+  const std::vector<Context *> cs = {&c};
+  if (const std::vector<ResidentLaunch> plan = resident_plan<R, LINK>(cs, runs); !plan.empty()) {
+    {
+      ResidentShare share(c.device, (double)plan[0].total / c.ws->num_cu);
+      rc = resident_launch<R, LINK>(cs, runs, plan[0]);
+      if (!rc) rc = bms_finish<R, LINK>(c, br, x, iters_out, x32, asm_fp32, rs);
+      if (rc < 0) hipStreamSynchronize(c.stream);  // nothing of it in flight when the share is given back
+    }
+    if (rc != kResidentGaveUp) return rc;
+    c.ws->resident_off = true;
+    br = BasisRun();
+    rc = bms_setup<R, LINK>(c, br, b, nrhs, nshift, shifts, res_abs, max_iter, iterc, tol_abs, tol_rel);
+    if (rc) return rc;
+  }
   GraphSlot &gs = c.ws->bms_graph[sizeof(R) == 8 ? 1 : 0];
   BmsGraphKey key;
   const std::vector<const int *> active = {br.a.active};
@@ -2941,19 +3175,47 @@ static int ms_cg_basis_group(std::vector<Context *> &cs, std::vector<GroupJob> &
   std::vector<BasisRun> runs(n);
   int nmin = 1 << 30;
   long cap_max = 0;
-  for (int l = 0; l < n; l++) {
-    GroupJob &j = jobs[l];
-    const int rc = bms_setup<R, LINK>(*cs[l], runs[l], j.b, j.nrhs, j.nshift, j.shifts, j.res_abs, j.max_iter, iterc);
-    if (rc) return rc;
-    BasisRun &br = runs[l];
-    br.timed = false;
-    for (DsArgs *d : {&br.hop, &br.mdm}) {
-      d->clk = nullptr;
-      d->clk_wg = nullptr;
-      d->clk_prev = nullptr;
+  auto setup = [&]() -> int {
+    for (int l = 0; l < n; l++) {
+      GroupJob &j = jobs[l];
+      runs[l] = BasisRun();
+      const int rc = bms_setup<R, LINK>(*cs[l], runs[l], j.b, j.nrhs, j.nshift, j.shifts, j.res_abs, j.max_iter, iterc);
+      if (rc) return rc;
+      BasisRun &br = runs[l];
+      br.timed = false;
+      for (DsArgs *d : {&br.hop, &br.mdm}) {
+        d->clk = nullptr;
+        d->clk_wg = nullptr;
+        d->clk_prev = nullptr;
+      }
+      nmin = std::min(nmin, j.nrhs);
+      cap_max = std::max(cap_max, br.cap);
     }
-    nmin = std::min(nmin, j.nrhs);
-    cap_max = std::max(cap_max, br.cap);
+    return 0;
+  };
+  auto finish = [&]() -> int {
+    for (int l = 0; l < n; l++) {
+      GroupJob &j = jobs[l];
+      j.out.iters = 0;
+      j.out.rc = bms_finish<R, LINK>(*cs[l], runs[l], j.x, &j.out.iters, j.x32, j.asm_fp32, &j.out.rs);
+      if (j.out.rc < 0 || j.out.rc == kResidentGaveUp) return j.out.rc;
+    }
+    return 0;
+  };
+  if (const int rc = setup()) return rc;
+  if (const std::vector<ResidentLaunch> plan = resident_plan<R, LINK>(cs, runs); !plan.empty()) {
+    int rc = 0;
+    {
+      unsigned most = 0;
+      for (const ResidentLaunch &rl : plan) most = std::max(most, rl.total);
+      ResidentShare share(c0.device, std::min(1.0, (double)most / c0.ws->num_cu));
+      for (size_t q = 0; q < plan.size() && !rc; q++) rc = resident_launch<R, LINK>(cs, runs, plan[q]);
+      if (!rc) rc = finish();
+      if (rc) hipStreamSynchronize(c0.stream);
+    }
+    if (rc != kResidentGaveUp) return rc;
+    c0.ws->resident_off = true;
+    if ((rc = setup())) return rc;
   }
   // the shape candidates run iteration 1 and read the iteration counter: on a
   // fresh lead context it still holds 0, for which the operands would be the
@@ -3001,13 +3263,7 @@ static int ms_cg_basis_group(std::vector<Context *> &cs, std::vector<GroupJob> &
   };
   auto chunk = [&](bool) -> bool { return chunk_run(c0, gs, false, key, sizeof(key), launch); };
   if (bms_iterate(c0, iterc, active, cap_max, chunk)) return -1;
-  for (int l = 0; l < n; l++) {
-    GroupJob &j = jobs[l];
-    j.out.iters = 0;
-    j.out.rc = bms_finish<R, LINK>(*cs[l], runs[l], j.x, &j.out.iters, j.x32, j.asm_fp32, &j.out.rs);
-    if (j.out.rc < 0) return -1;
-  }
-  return 0;
+  return finish();
 }
 
 // r^(K) of a continued system (basis slot K, precision R) as an FP64 source

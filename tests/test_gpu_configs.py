@@ -684,3 +684,77 @@ def test_graph_capture_once_per_solve_shape():
     assert counts[4] == counts[1]
     for x in sols[1:]:
         assert np.array_equal(x, sols[0])
+
+
+# ----------------------------------------- small lattices: one-launch solves
+@pytest.mark.parametrize("dims,n_pf", [((4, 4, 4, 4), 1), ((6, 4, 4, 6), 3), ((6, 6, 6, 6), 1), ((6, 6, 6, 6), 2),
+                                       ((8, 8, 8, 4), 8), ((20, 14, 12, 6), 2), ((20, 14, 12, 6), 4),
+                                       ((16, 16, 16, 16), 1), ((16, 16, 16, 16), 3), ((18, 16, 16, 16), 1),
+                                       ((24, 24, 24, 8), 1)])
+def test_one_launch_solves(dims, n_pf, monkeypatch):
+    """Multi-shift solves whose iterations run as one launch, over the forms
+    that launch takes: one workgroup and a partly filled one, systems split
+    over members and together (1, 2, 4 per member), odd V/16 (slots that are no
+    whole cache lines in FP32 for an odd number of systems), 256 and 512
+    lanes, two sites per lane.  FP64 solutions agree with the launches per
+    iteration (RHMC_DSLASH_NR set) to 1e-9, the true residuals meet 1e-10 |b|;
+    FP32 ones to 2e-4 and 2e-5 (both stop at 1e-6, on recurrences that round
+    differently); iteration counts are the same in FP64, a repeated solve is
+    the same bit for bit."""
+    mass = 0.05
+    lat = fields.Lattice(*dims)
+    U = fields.random_links(lat, 31, 0.3)
+    phi = fields.gauss_spinor(lat, 32, n_pf)
+    b = np.geomspace(1e-4, 2.0, 7)
+    bn = np.linalg.norm(phi.reshape(n_pf, -1), axis=1)
+    say("one-launch solve", dims, n_pf)
+    out = {}
+    for mode in ("one", "many"):
+        if mode == "many":
+            monkeypatch.setenv("RHMC_DSLASH_NR", "1")
+        g = Gpu(dims, mass=mass, n_pf=n_pf, max_order=7)
+        g.init0(U)
+        g.init1(phi=phi)
+        for prec, res in ((0, 1e-10), (2, 1e-6)):
+            # the first solve may fill the initial basis, after which its
+            # capacity follows the iterations needed
+            g.multishift(b, res, relative=True, precision=prec)
+            it = g.multishift(b, res, relative=True, precision=prec)
+            x = g.get_fermions("smf")
+            rn = g.shifted_residuals(b) / bn[:, None]
+            assert rn.max() <= (1e-10 if prec == 0 else 2e-5)
+            g.multishift(b, res, relative=True, precision=prec)
+            assert np.array_equal(g.get_fermions("smf"), x)
+            out[mode, prec] = (it, x)
+        g.close()
+    assert out["one", 0][0] == out["many", 0][0]
+    for prec, tol in ((0, 1e-9), (2, 2e-4)):
+        for x, y in zip(out["one", prec][1], out["many", prec][1]):
+            assert rel(x, y) < tol
+
+
+@pytest.mark.parametrize("precision", [0, 2])
+def test_one_launch_solve_that_gives_up(precision, monkeypatch):
+    """A one-launch solve whose waits are bounded at 0 ticks leaves (every
+    workgroup exits) and the solve is repeated with the launches per
+    iteration: the same status and solutions as without it."""
+    dims, mass = (16, 16, 16, 16), 0.05
+    lat = fields.Lattice(*dims)
+    U = fields.random_links(lat, 33, 0.3)
+    phi = fields.gauss_spinor(lat, 34, 1)
+    b = np.geomspace(1e-4, 2.0, 7)
+    say("one-launch solve, no wait", precision)
+    xs = []
+    for wait in ("0", None):
+        if wait is None:
+            monkeypatch.delenv("RHMC_RESIDENT_WAIT")
+        else:
+            monkeypatch.setenv("RHMC_RESIDENT_WAIT", wait)
+        g = Gpu(dims, mass=mass, n_pf=1, max_order=7)
+        g.init0(U)
+        g.init1(phi=phi)
+        for _ in range(2):
+            g.multishift(b, 1e-10 if precision == 0 else 1e-6, relative=True, precision=precision)
+        xs.append(g.get_fermions("smf"))
+        g.close()
+    assert rel(xs[0], xs[1]) < (1e-9 if precision == 0 else 2e-4)
