@@ -555,4 +555,95 @@ __global__ __launch_bounds__(64 * kResMaxWaves) __attribute__((amdgpu_waves_per_
   }
 }
 
+// ---- power iterations of a small lattice: n of them per launch on the FP64
+// 12-real links, p <- (pa p + pb hop(hop(p)/2)) / |p|, meeting twice per
+// iteration as the solver does (the first time without a sum).  p of
+// iteration i is in slot (base + i) mod (n + 1) of r.basis, h in slot i of
+// r.h, so no slot is read before it is written in a launch.  norms[0] is
+// |p|^2 at the start, norms[i] that of iteration i, norms[n+1] the
+// iterations run (-1: the grid gave up); the launch ends at the first one
+// whose norm changed by at most tol relatively.
+struct PowArgs {
+  ResArgs r;
+  double pa, pb, tol;
+  double *norms;
+  int n, base;
+  long long wait;
+};
+
+template <int P>
+__global__ __launch_bounds__(64 * kResMaxWaves) __attribute__((amdgpu_waves_per_eu(2))) void k_pow_resident(PowArgs q) {
+  using C = double2;
+  constexpr int LINK = LINK_D12;
+  const ResArgs &a = q.r;
+  __shared__ ResShared<1> s;
+  const int copy = (int)(blockIdx.x & 7u);
+  const int wg = (int)((blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3));
+  if (wg >= a.nwg) return;
+  const long Vh = a.L.Vh;
+  const int mu = threadIdx.x & 3, nw = blockDim.x >> 6, spw = blockDim.x >> 2;
+  bool mine[P];
+  unsigned own[P];
+  ResHop<double> odd[P], even[P];
+  C pv[P];
+  C *ring = (C *)a.basis;
+#pragma unroll
+  for (int p = 0; p < P; p++) {
+    const int site = (wg * P + p) * spw + (int)(threadIdx.x >> 2);
+    const bool valid = site < (int)Vh;
+    const int h = valid ? site : (int)Vh - 1;
+    mine[p] = valid && mu < 3;
+    own[p] = (unsigned)((mu < 3 ? mu : 2) * Vh + h);
+    res_hop_setup<double, LINK>(a, 1, h, mu, odd[p]);
+    res_hop_setup<double, LINK>(a, 0, h, mu, even[p]);
+    pv[p] = ring[(long)q.base * a.stride + own[p]];
+  }
+  if (threadIdx.x == 0) s.aborted = 0;
+  ResLinks<double, LINK> lo, le;
+  if constexpr (P == 1) {
+    res_links<double, LINK>(a, odd[0], lo);
+    res_links<double, LINK>(a, even[0], le);
+  }
+  __syncthreads();
+  double n2 = q.norms[0], prev = sqrt(n2);
+  int i = 0;
+  for (bool met = false; i < q.n && !met; i++) {
+    const C *in = ring + (long)((q.base + i) % (q.n + 1)) * a.stride;
+    C *out = ring + (long)((q.base + i + 1) % (q.n + 1)) * a.stride, *hs = (C *)a.h + (long)i * a.stride;
+    double v[1] = {0.0};
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+      if constexpr (P == 1) res_keep(lo);
+      else res_links<double, LINK>(a, odd[p], lo);
+      C o[1];
+      res_hop<double, LINK, 1>(odd[p], lo, in, Vh, 0, 1, mu, o);
+      if (mine[p]) res_put(hs + own[p], cscale(o[0], 0.5));
+    }
+    res_arrive<1>(a, s, wg, 2 * i, v);
+    if (!res_wait<1>(a, s, wg, copy, q.wait, 2 * i)) break;
+    const double sc = 1.0 / sqrt(n2), pa = q.pa * sc, pb = q.pb * sc;
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+      if constexpr (P == 1) res_keep(le);
+      else res_links<double, LINK>(a, even[p], le);
+      C o[1];
+      res_hop<double, LINK, 1>(even[p], le, hs, Vh, 0, 1, mu, o);
+      pv[p] = make_double2(fmar(pa, pv[p].x, pb * o[0].x), fmar(pa, pv[p].y, pb * o[0].y));
+      if (mine[p]) {
+        res_put(out + own[p], pv[p]);
+        v[0] += pv[p].x * pv[p].x + pv[p].y * pv[p].y;
+      }
+    }
+    res_arrive<1>(a, s, wg, 2 * i + 1, v);
+    if (!res_wait<1>(a, s, wg, copy, q.wait, 2 * i + 1)) break;
+    n2 = 0.0;
+    for (int k = 0; k < nw; k++) n2 += s.wave[1][k][0];
+    if (wg == 0 && threadIdx.x == 0) q.norms[i + 1] = n2;
+    const double norm = sqrt(n2);
+    met = !(fabs(prev - norm) / norm > q.tol);
+    prev = norm;
+  }
+  if (wg == 0 && threadIdx.x == 0) q.norms[q.n + 1] = s.aborted ? -1.0 : (double)i;
+}
+
 }  // namespace rhmc

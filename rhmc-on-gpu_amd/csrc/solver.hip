@@ -471,8 +471,9 @@ __device__ __forceinline__ double block_sum_partials(const double *p, int n) {
 }
 
 // ------------------------------------------------------------------ Dslash
-// DS_BMS: the stored-basis solver's M^dag M with the residual update
-enum DsMode { DS_HOP = 0, DS_MDAGM = 1, DS_RESID = 2, DS_BMS = 3 };
+// DS_BMS: the stored-basis solver's M^dag M with the residual update;
+// DS_POW: the power iteration's, normalising its operand
+enum DsMode { DS_HOP = 0, DS_MDAGM = 1, DS_RESID = 2, DS_BMS = 3, DS_POW = 4 };
 enum DsRed { RED_NONE = 0, RED_DOT = 1, RED_NORM = 2 };
 enum LinkFmt { LINK_D18 = 0, LINK_S12 = 1, LINK_D12 = 2 };
 
@@ -521,6 +522,10 @@ struct DsArgs {
   BmsShared *bms; const double *bms_part; int bms_nbr;
   MsState *bms_ms; BmsHist *bms_hist; int *bms_active; int bms_cap, bms_nshift;
   const double *bms_hpart; int bms_hnbr;
+  // DS_POW: out = (pow_a pin + pow_b hop(in)) / |pin|, |pin|^2 the sum of the
+  // partials of the launch that wrote pin (bms_hpart, bms_hnbr of them),
+  // which the first workgroup also stores in pow_norm
+  double pow_a, pow_b; double *pow_norm;
   RedArgs red;
 };
 
@@ -653,6 +658,13 @@ __device__ __forceinline__ void bms_alpha(const DsArgs &a, int jbase, unsigned s
     }
   }
   __syncthreads();
+}
+
+// DS_POW, every workgroup: 1 / |pin| (a fixed-order sum, the same in all)
+__device__ __forceinline__ double pow_scale(const DsArgs &a, unsigned sb) {
+  const double n2 = block_sum_partials(a.bms_hpart, a.bms_hnbr);
+  if (sb == 0 && threadIdx.x == 0) *a.pow_norm = n2;
+  return 1.0 / sqrt(n2);
 }
 
 __device__ __forceinline__ unsigned long long *clk_slot(const DsArgs &a) {
@@ -858,7 +870,7 @@ constexpr int ds_waves() {
 // stored-basis solver's DS_BMS output is ds_site_out_bms).
 template <typename R, int NR, int MODE, int RED>
 __device__ __forceinline__ void ds_site_out(const DsArgs &a, const Cx<R> (&acc)[NR][3], const bool (&act)[NR],
-                                            double (&red)[NR], int jbase, int h, const Cx<R> *pinb) {
+                                            double (&red)[NR], int jbase, int h, const Cx<R> *pinb, R scale) {
   using C = Cx<R>;
   const long Vh = a.L.Vh;
 #pragma unroll
@@ -870,6 +882,15 @@ __device__ __forceinline__ void ds_site_out(const DsArgs &a, const Cx<R> (&acc)[
     if (MODE == DS_HOP) {
 #pragma unroll
       for (int i = 0; i < 3; i++) res[i] = cscale(acc[r][i], (R)0.5);
+    } else if (MODE == DS_POW) {
+      const R pa = (R)a.pow_a * scale, pb = (R)a.pow_b * scale;
+      const C *p = pinb + (long)j * a.pin_vs + h;
+#pragma unroll
+      for (int i = 0; i < 3; i++) {
+        const C pv = p[(long)i * Vh];
+        res[i].x = fmar(pa, pv.x, pb * acc[r][i].x);
+        res[i].y = fmar(pa, pv.y, pb * acc[r][i].y);
+      }
     } else {
       const R d = (R)a.diag[j];
       const C *p = pinb + (long)j * a.pin_vs + h;
@@ -967,6 +988,7 @@ __device__ __forceinline__ void ds_body(const DsArgs &a, unsigned bid, unsigned 
   const int jbase = ch * NR;
   __shared__ R bab[2][NR];
   if (MODE == DS_BMS) bms_alpha<R, NR>(a, jbase, sb, bab);
+  const R scale = MODE == DS_POW ? (R)pow_scale(a, sb) : (R)1;
   const bool rk_ok = MODE == DS_BMS && *a.iterp + a.iter_off + 1 < a.bms_cap;
   // iteration k >= 2 of the stored-basis solver reads basis slot k-2 too
   const bool use_prev = MODE == DS_BMS && *a.iterp + a.iter_off + 1 >= 2;
@@ -1032,7 +1054,7 @@ __device__ __forceinline__ void ds_body(const DsArgs &a, unsigned bid, unsigned 
       if constexpr (!kBmsEarly) bms_site_loads<R, NR>(a, jbase, h, pinb, use_prev, pv, qv);
       ds_site_out_bms<R, NR>(a, acc, act, red, jbase, h, pinb, bab, rk_ok, pv, qv);
     }
-    else ds_site_out<R, NR, MODE, RED>(a, acc, act, red, jbase, h, pinb);
+    else ds_site_out<R, NR, MODE, RED>(a, acc, act, red, jbase, h, pinb, scale);
   }
   if (RED != RED_NONE) block_partials<NR>(red, a.red.partial, jbase, a.nvec, a.nsb, sb);
   clk_end(a, bid);
@@ -1167,6 +1189,7 @@ __device__ __forceinline__ void ds_ls_body(const DsArgs &a, unsigned bid, unsign
   const int jbase = ch * NR;
   __shared__ R bab[2][NR];
   if (MODE == DS_BMS) bms_alpha<R, NR>(a, jbase, sb, bab);
+  const R scale = MODE == DS_POW ? (R)pow_scale(a, sb) : (R)1;
   const bool rk_ok = MODE == DS_BMS && *a.iterp + a.iter_off + 1 < a.bms_cap;
   const bool use_prev = MODE == DS_BMS && *a.iterp + a.iter_off + 1 >= 2;
   const int nunits = a.ntiles * (kBlock / kLsSites);
@@ -1239,6 +1262,11 @@ __device__ __forceinline__ void ds_ls_body(const DsArgs &a, unsigned bid, unsign
       C res;
       if (MODE == DS_HOP) {
         res = cscale(av, (R)0.5);
+      } else if (MODE == DS_POW) {
+        const C pv = (pinb + (long)j * a.pin_vs + h)[(long)col * Vh];
+        const R pa = (R)a.pow_a * scale, pb = (R)a.pow_b * scale;
+        res.x = fmar(pa, pv.x, pb * av.x);
+        res.y = fmar(pa, pv.y, pb * av.y);
       } else {
         const C pv = (pinb + (long)j * a.pin_vs + h)[(long)col * Vh];
         const R d = (R)a.diag[j];
@@ -1496,6 +1524,11 @@ static void dslash_launch(Context &c, DsArgs &a, int code) {
   const int nr = shape_nr(code), lanes = shape_lanes(code) == 4 ? 4 : 1;
   dslash_prep<MODE, RED>(c, a, code);
   dim3 grid(a.nsb * a.nch);
+  if constexpr (MODE == DS_POW) {  // one vector
+    if (lanes == 4) DS_LAUNCH((k_dslash_ls<R, LINK, 1, MODE, RED>));
+    else DS_LAUNCH((k_dslash<R, LINK, 1, MODE, RED>));
+    return;
+  }
   if (lanes == 4) {
     switch (nr) {
       case 8: DS_LAUNCH((k_dslash_ls<R, LINK, 8, MODE, RED>)); break;
@@ -3782,28 +3815,6 @@ int vec_norms2(Context &c, const double2 *v, int nvec, long vs, double *out) {
   return d2h_sync(c, out, sums, sizeof(double) * nvec) ? 0 : -1;
 }
 
-// p = a*r - p
-__global__ __launch_bounds__(kBlock) void k_axmy(double2 *p, const double2 *r, double a, long n) {
-  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) {
-    const double2 rv = r[i];
-    double2 pv = p[i];
-    pv.x = a * rv.x - pv.x;
-    pv.y = a * rv.y - pv.y;
-    p[i] = pv;
-  }
-}
-
-// r = p / sqrt(*n2) (the norm of the previous iteration, read on the device)
-__global__ __launch_bounds__(kBlock) void k_scale_by_norm(double2 *r, const double2 *p, const double *n2, long n) {
-  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) {
-    const double s = 1.0 / sqrt(*n2);
-    const double2 v = p[i];
-    r[i] = make_double2(s * v.x, s * v.y);
-  }
-}
-
 // |v|^2 of one vector into *dst on the device (no host round trip)
 static void norm2_to(Context &c, const double2 *v, long n, double *dst) {
   RedArgs red = make_red(c, 1, EPI_STORE, nullptr, dst);
@@ -3816,62 +3827,132 @@ static void norm2_to(Context &c, const double2 *v, long n, double *dst) {
 // Power iterations of findminmax.cc:12-137 in FP64: p <- A r with r =
 // p / |p|, A = M^dag M (largest eigenvalue |A r| at convergence) or
 // max - M^dag M (then min = max - |A r|), until the relative change of |p|
-// is at most tol.  Every iteration stores |p|^2 on the device and
-// normalises with it there; the host reads the norms after each chunk of
-// kPowChunk iterations and stops at the first iteration that met the test,
-// whose value it returns (the chunk's later iterations are discarded), so
-// the result is the one a test after every iteration gives, without a
-// host round trip per iteration.
+// is at most tol, at most kPowMax times.  Since A is linear the operand is
+// not normalised first: h = D_oe p is a plain hop and the second launch
+// (DS_POW) scales with 1/|p| from the partials of the launch before, so an
+// iteration is two launches on the 12-real links of the FP64 solves (five or
+// six launches with separate scaling, difference and norms on 18-real links
+// took 68 us per iteration at 32^3x8, these 45).  Small lattices run kPowSmall
+// iterations per launch (k_pow_resident; 8^3x4: 22 -> 5.1 us per iteration).
+// The host reads the norms chunk by chunk and stops at the first iteration
+// that met the test, whose value it returns (later iterations are
+// discarded), so the result is the one a test after every iteration gives,
+// without a host round trip per iteration.
 constexpr int kPowChunk = 8;
 constexpr int kPowMax = 20000;
+constexpr int kPowSmall = 64;
+
+// the first of iterations i0 .. i0+n-1 that meets the test, given their norms
+// |p|^2 in h[1..n] (h[0]: of iteration i0-1); 0 if none does
+static int power_met(const double *h, int i0, int n, double tol, double &norm) {
+  for (int q = 1; q <= n && i0 + q - 1 <= kPowMax; q++) {
+    const double prev = sqrt(h[q - 1]);
+    norm = sqrt(h[q]);
+    if (!(fabs(prev - norm) / norm > tol) || i0 + q - 1 == kPowMax) return i0 + q - 1;
+  }
+  return 0;
+}
+
+// small lattices; returns 0 done, 1 not taken (or given up: use the launches)
+static int power_resident(Context &c, const double2 *start, double tol, double pa, double pb, double *norm,
+                          int *loops) {
+  Workspace *w = c.ws;
+  if (w->resident_off || w->num_cu < 8 || getenv("RHMC_DSLASH_NR")) return 1;
+  int threads = 256, sites = 1, nwg = 0;
+  unsigned total = resident_wgs(c, threads, sites, nwg);
+  if (total > (unsigned)w->num_cu) total = resident_wgs(c, threads = 512, sites, nwg);
+  if (total > (unsigned)w->num_cu) total = resident_wgs(c, threads, sites = 2, nwg);
+  if (total > (unsigned)w->num_cu) return 1;
+  const long n = 3 * c.Vh;  // whole cache lines: V/2 is a multiple of 8
+  double2 *p = (double2 *)ws_get(c, S_PW1, sizeof(double2) * n * (2 * kPowSmall + 1));
+  double *pn = (double *)ws_get(c, S_PWN, sizeof(double) * (kPowSmall + 2));
+  const int np = kResRing * kResCopies * res_copy(nwg);
+  unsigned long long *part = (unsigned long long *)ws_get(c, S_RES_PART, sizeof(unsigned long long) * np + 64);
+  if (!p || !pn || !part) return -1;
+  hipMemcpyAsync(p, start, sizeof(double2) * n, hipMemcpyDeviceToDevice, c.stream);
+  norm2_to(c, p, n, pn);
+  PowArgs a = {};
+  a.r.L = c.L;
+  a.r.U = c.U64c;
+  a.r.basis = p;
+  a.r.h = p + (kPowSmall + 1) * n;
+  a.r.stride = n;
+  a.r.part = part;
+  a.r.abort = (int *)(part + np);
+  a.r.nvec = 1;
+  a.r.nwg = nwg;
+  a.pa = pa; a.pb = pb; a.tol = tol;
+  a.norms = pn; a.n = kPowSmall;
+  const char *wait = getenv("RHMC_RESIDENT_WAIT");
+  a.wait = wait ? atoll(wait) : kResWaitTicks;
+  ResidentShare share(c.device, (double)total / w->num_cu);
+  double h[kPowSmall + 2];
+  for (int i0 = 1;; i0 += kPowSmall) {
+    hipLaunchKernelGGL(k_res_init, dim3(std::min(256, (np + kBlock - 1) / kBlock)), dim3(kBlock), 0, c.stream, part,
+                       np, a.r.abort);
+    if (sites == 1) hipLaunchKernelGGL(k_pow_resident<1>, dim3(total), dim3(threads), 0, c.stream, a);
+    else hipLaunchKernelGGL(k_pow_resident<2>, dim3(total), dim3(threads), 0, c.stream, a);
+    if (!d2h_sync(c, h, pn, sizeof(double) * (kPowSmall + 2))) return -1;
+    const int ran = (int)h[kPowSmall + 1];
+    if (ran < 0) {
+      w->resident_off = true;
+      return 1;
+    }
+    if ((*loops = power_met(h, i0, ran, tol, *norm))) return 0;
+    // the last vector, in its slot of the ring, is the next launch's first
+    a.base = (a.base + kPowSmall) % (kPowSmall + 1);
+    hipMemcpyAsync(pn, pn + kPowSmall, sizeof(double), hipMemcpyDeviceToDevice, c.stream);
+  }
+}
+
 static int power_iter(Context &c, const double2 *start, double tol, int is_min, double mx, double *out, int *loops) {
   const long Vh = c.Vh, n = 3 * Vh;
-  double2 *p = (double2 *)ws_get(c, S_PW1, sizeof(double2) * n);
-  double2 *r = (double2 *)ws_get(c, S_PW2, sizeof(double2) * n);
-  double2 *hh = (double2 *)ws_get(c, S_PW3, sizeof(double2) * n);
-  double *diag = (double *)ws_get(c, S_DIAG, sizeof(double) * 256);
-  double *pn = (double *)ws_get(c, S_PWN, sizeof(double) * (kPowMax + kPowChunk + 1));
-  if (!p || !r || !hh || !diag || !pn) return -1;
-  hipMemcpyAsync(p, start, sizeof(double2) * n, hipMemcpyDeviceToDevice, c.stream);
   const double m2 = c.mass * c.mass;
-  if (!h2d(c, diag, &m2, sizeof(double))) return -1;
-  norm2_to(c, p, n, pn);  // pn[0] = |start|^2
-  const unsigned nb = (unsigned)((n + kBlock - 1) / kBlock);
-  double prev = -1.0, norm = 0.0;
+  // M^dag M p = m^2 p - hop(h)/2, h = D_oe p
+  const double pa = is_min ? mx - m2 : m2, pb = is_min ? 0.5 : -0.5;
+  double norm = 0.0;
+  const int small = power_resident(c, start, tol, pa, pb, &norm, loops);
+  if (small < 0) return -1;
+  if (small == 0) {
+    *out = is_min ? mx - norm : norm;
+    return 0;
+  }
+  double2 *p[2] = {(double2 *)ws_get(c, S_PW1, sizeof(double2) * n), (double2 *)ws_get(c, S_PW2, sizeof(double2) * n)};
+  double2 *hh = (double2 *)ws_get(c, S_PW3, sizeof(double2) * n);
+  double *pn = (double *)ws_get(c, S_PWN, sizeof(double) * (kPowChunk + 1));
+  const size_t pb_bytes = sizeof(double) * nbx_of(c);
+  double *part[2] = {(double *)ws_get(c, S_PARTIAL2, pb_bytes), (double *)ws_get(c, S_HPART, pb_bytes)};
+  if (!p[0] || !p[1] || !hh || !pn || !part[0] || !part[1]) return -1;
+  hipMemcpyAsync(p[0], start, sizeof(double2) * n, hipMemcpyDeviceToDevice, c.stream);
+  // partials of |p|^2: those of the launch that wrote p
+  RedArgs red = make_red(c, 1, EPI_STORE, nullptr, nullptr);
+  red.nbr = (int)reduce_blocks(c, 1);
+  red.partial = part[0];
+  hipLaunchKernelGGL(k_norms, dim3(red.nbr, 1), dim3(kBlock), 0, c.stream, p[0], n, Vh, 1, red);
   double h[kPowChunk + 1];
-  int done = 0;
-  for (int i0 = 1; !done && i0 <= kPowMax; i0 += kPowChunk) {
+  for (int i0 = 1;; i0 += kPowChunk) {
     for (int i = i0; i < i0 + kPowChunk; i++) {
-      hipLaunchKernelGGL(k_scale_by_norm, dim3(nb), dim3(kBlock), 0, c.stream, r, p, pn + i - 1, n);
-      launch_hop_d(c, 1, r, hh, 1, n, n);
+      const int o = (i - 1) & 1;
+      launch_hop_d12(c, 1, p[o], hh, 1, n, n);
       DsArgs a = {};
-      a.par_out = 0; a.U = c.U64; a.in = hh; a.in_vs = n; a.out = p; a.out_vs = n; a.pin = r; a.pin_vs = n;
-      a.diag = diag; a.nvec = 1;
-      if (!is_min) {
-        a.red = make_red(c, 1, EPI_STORE, nullptr, pn + i);
-        dslash_dispatch<double, LINK_D18, DS_MDAGM, RED_NORM>(c, a);
-        finalize(c, a.red, 1, false);
-      } else {
-        dslash_dispatch<double, LINK_D18, DS_MDAGM, RED_NONE>(c, a);
-        hipLaunchKernelGGL(k_axmy, dim3(nb), dim3(kBlock), 0, c.stream, p, r, mx, n);
-        norm2_to(c, p, n, pn + i);
-      }
+      a.par_out = 0; a.U = c.U64c; a.in = hh; a.in_vs = n; a.out = p[1 - o]; a.out_vs = n; a.pin = p[o]; a.pin_vs = n;
+      a.nvec = 1;
+      a.pow_a = pa; a.pow_b = pb; a.pow_norm = pn + i - i0;
+      a.bms_hpart = part[o]; a.bms_hnbr = red.nbr;
+      a.red = red;
+      a.red.partial = part[1 - o];
+      dslash_dispatch<double, LINK_D12, DS_POW, RED_NORM>(c, a);
+      red.nbr = a.red.nbr;
     }
-    if (!d2h_sync(c, h, pn + i0 - 1, sizeof(double) * (kPowChunk + 1))) return -1;
-    if (prev < 0.0) prev = sqrt(h[0]);
-    for (int q = 1; q <= kPowChunk && i0 + q - 1 <= kPowMax; q++) {
-      norm = sqrt(h[q]);
-      const double rel = fabs(prev - norm) / norm;
-      prev = norm;
-      if (!(rel > tol) || i0 + q - 1 == kPowMax) {
-        *loops = i0 + q - 1;
-        done = 1;
-        break;
-      }
-    }
+    RedArgs last = red;
+    last.partial = part[(i0 + kPowChunk - 1) & 1];
+    last.sums = pn + kPowChunk;
+    finalize(c, last, 1, false);
+    if (!d2h_sync(c, h, pn, sizeof(double) * (kPowChunk + 1))) return -1;
+    if ((*loops = power_met(h, i0, kPowChunk, tol, norm))) break;
   }
   *out = is_min ? mx - norm : norm;
-  return hip_ok(c, hipStreamSynchronize(c.stream), "power") ? 0 : -1;
+  return hip_ok(c, hipGetLastError(), "power") ? 0 : -1;
 }
 
 int power_max(Context &c, const double2 *start, double tol, double *out, int *loops) {

@@ -758,3 +758,27 @@ def test_one_launch_solve_that_gives_up(precision, monkeypatch):
         xs.append(g.get_fermions("smf"))
         g.close()
     assert rel(xs[0], xs[1]) < (1e-9 if precision == 0 else 2e-4)
+
+
+@pytest.mark.parametrize("dims", [(4, 4, 4, 4), (6, 4, 4, 6), (6, 6, 6, 6), (20, 14, 12, 6), (16, 16, 16, 16),
+                                  (18, 16, 16, 16), (24, 24, 24, 12)])
+def test_power_iterations_in_one_launch(dims, monkeypatch):
+    """The power iterations of small lattices (64 per launch, one or two sites
+    per lane; several launches each) stop at the same iteration as the two
+    launches per iteration (RHMC_DSLASH_NR set; 24^3x12 always runs those):
+    both bounds equal to 1e-11 of the largest eigenvalue, the rounding of
+    a few hundred normalised applications (1e-16 each)."""
+    lat = fields.Lattice(*dims)
+    g = Gpu(dims, mass=0.05)
+    g.init0(fields.random_links(lat, 41, 0.3))
+    say("power iterations", dims)
+    got = []
+    for many in (False, True):
+        if many:
+            monkeypatch.setenv("RHMC_DSLASH_NR", "1")
+        mx = g.find_max(1e-5, seed=5)
+        got.append((mx, g.find_min(mx, 1e-5, seed=6)))
+    say(got)
+    assert abs(got[0][0] - got[1][0]) < 1e-11 * got[1][0]
+    assert abs(got[0][1] - got[1][1]) < 1e-11 * got[1][0]
+    g.close()
