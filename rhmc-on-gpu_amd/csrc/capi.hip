@@ -106,12 +106,13 @@ int gpu_create(const rhmc_gpu_params *p, rhmc_gpu_t *out) {
   Context &c = h->c;
   c.device = p->device;
   if (!hip_ok(c, hipSetDevice(p->device), "hipSetDevice")) { delete h; return RHMC_EHIP; }
+  host_stage_retain();
   fill_dims(c, p->nx, p->ny, p->nz, p->nt, p->antiperiodic_t);
   c.mass = p->mass;
   c.beta = p->beta;
   c.n_pf = p->n_pf;
   c.max_order = p->max_order;
-  if (!hip_ok(c, hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking), "stream")) { delete h; return RHMC_EHIP; }
+  if (!hip_ok(c, hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking), "stream")) { gpu_destroy(h); return RHMC_EHIP; }
   const long Vh = c.Vh;
   c.U64 = (double2 *)dev_alloc(c, sizeof(double2) * 72 * Vh);
   c.U64_save = (double2 *)dev_alloc(c, sizeof(double2) * 72 * Vh);
@@ -154,6 +155,7 @@ int gpu_destroy(rhmc_gpu_t h) {
   kernel_timing_release(c);
   workspace_destroy(c.ws);
   if (c.stream) hipStreamDestroy(c.stream);
+  host_stage_release();
   delete h;
   return RHMC_OK;
 }

@@ -782,3 +782,44 @@ def test_power_iterations_in_one_launch(dims, monkeypatch):
     assert abs(got[0][0] - got[1][0]) < 1e-11 * got[1][0]
     assert abs(got[0][1] - got[1][1]) < 1e-11 * got[1][0]
     g.close()
+
+
+# ------------------------------------------------- large host transfers
+@pytest.mark.parametrize("dims", [(8, 8, 8, 4), (16, 14, 12, 6), (18, 16, 14, 10), (32, 32, 16, 8)])
+def test_host_transfers_round_trip(dims):
+    """Links, momenta, force and pseudofermions go to the device and come back
+    bit for bit, below and above the size that is moved in chunks (8 MB; the
+    last chunk partly filled), also with two handles transferring from two
+    threads at once."""
+    import threading
+    lat = fields.Lattice(*dims)
+    say("transfers", dims)
+    err = []
+
+    def work(seed):
+        try:
+            U = fields.random_links(lat, seed, 0.3)
+            P = fields.gauss_momenta(lat, seed + 1)
+            F = 1j * fields.gauss_momenta(lat, seed + 2)
+            phi = fields.gauss_spinor(lat, seed + 3, 2)
+            g = Gpu(dims, mass=0.1, n_pf=2, max_order=2)
+            for _ in range(2):
+                g.init0(U)
+                g.init1(phi=phi, ipdot=F, momenta=P)
+                U1, F1, P1 = g.end()
+                assert np.array_equal(U1, U)
+                # packed as 8 reals: the third diagonal entry is rebuilt
+                for a, b in ((P1, P), (F1, F)):
+                    assert np.array_equal(a[:, 0, 1:], b[:, 0, 1:]) and np.array_equal(a[:, 1, 2], b[:, 1, 2])
+                    assert np.abs(a - b).max() < 1e-14
+                assert np.array_equal(g.get_fermions("mf"), phi)
+            g.close()
+        except Exception as e:  # reported by the main thread
+            err.append(e)
+
+    th = [threading.Thread(target=work, args=(60 + 10 * k,)) for k in range(2)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not err, err
