@@ -251,82 +251,194 @@ int fermion_force_noalloc(Context &c, int order, const double *num, int accumula
 // staples.cc:16-74, ipdot.cc:25-79:
 //   ipdot_mu(x) = TA(U_mu(x) beta/3 sum_{nu!=mu} [U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
 //                                              + U_nu(x+mu-nu)^+ U_mu(x-nu)^+ U_nu(x-nu)])
-// one step along mu with the periodic wrap, no division
-__device__ __forceinline__ void step_coord(const LatticeDims &L, int &x, int &y, int &z, int &t, int mu, int d) {
-  if (mu == 0) x = d > 0 ? (x + 1 == L.nx ? 0 : x + 1) : (x == 0 ? L.nx - 1 : x - 1);
-  else if (mu == 1) y = d > 0 ? (y + 1 == L.ny ? 0 : y + 1) : (y == 0 ? L.ny - 1 : y - 1);
-  else if (mu == 2) z = d > 0 ? (z + 1 == L.nz ? 0 : z + 1) : (z == 0 ? L.nz - 1 : z - 1);
-  else t = d > 0 ? (t + 1 == L.nt ? 0 : t + 1) : (t == 0 ? L.nt - 1 : t - 1);
+// Links come from the FP64 12-real copy.  A staple is a product of three links,
+// each unitary with a known sign (its staggered phase), so it is unitary with
+// the product of the signs, and only its first two rows are multiplied out;
+// the third is rebuilt once from them, as it is for the links that are needed
+// whole: 369 complex products per link instead of 465.
+struct Rows {
+  double2 e[2][3];
+};
+// rows 0 and 1 of link mu at half index h of parity par
+__device__ __forceinline__ void rows_load(const double2 *U12, long Vh, int mu, int par, int h, Rows &m) {
+  const double2 *b = U12 + (long)(mu * 2 + par) * 6 * Vh;
+  const unsigned off = (unsigned)h * (unsigned)sizeof(double2);
+#pragma unroll
+  for (int k = 0; k < 6; k++) m.e[k / 3][k % 3] = ld_off(b + (long)k * Vh, off);
+}
+// the whole matrix, its sign (-1 for an odd number of phases) on row 2
+__device__ __forceinline__ Mat<double> rows_mat(const Rows &r, int odd) {
+  Mat<double> m;
+#pragma unroll
+  for (int k = 0; k < 6; k++) m.e[k / 3][k % 3] = r.e[k / 3][k % 3];
+  rebuild_row2(m, odd & 1 ? -1.0 : 1.0);
+  return m;
+}
+// rows of a b^+ and of a b
+__device__ __forceinline__ Rows rows_nd(const Rows &a, const Mat<double> &b) {
+  Rows r;
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      double2 s = cmul(a.e[i][0], cconj(b.e[j][0]));
+      cfma(s, a.e[i][1], cconj(b.e[j][1]));
+      cfma(s, a.e[i][2], cconj(b.e[j][2]));
+      r.e[i][j] = s;
+    }
+  return r;
+}
+__device__ __forceinline__ Rows rows_nn(const Rows &a, const Mat<double> &b) {
+  Rows r;
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      double2 s = cmul(a.e[i][0], b.e[0][j]);
+      cfma(s, a.e[i][1], b.e[1][j]);
+      cfma(s, a.e[i][2], b.e[2][j]);
+      r.e[i][j] = s;
+    }
+  return r;
+}
+// Ends a stage: the values pass through an empty asm statement (in-out
+// operands, memory clobber), so the stage's multiply-adds are issued after
+// the loads before it in program order and before those that follow.
+__device__ __forceinline__ void rows_fence(Rows &r) {
+#pragma unroll
+  for (int k = 0; k < 6; k++) asm volatile("" : "+v"(r.e[k / 3][k % 3].x), "+v"(r.e[k / 3][k % 3].y) : : "memory");
+}
+__device__ __forceinline__ void mat_fence(Mat<double> &m) {
+#pragma unroll
+  for (int k = 0; k < 9; k++) asm volatile("" : "+v"(m.e[k / 3][k % 3].x), "+v"(m.e[k / 3][k % 3].y) : : "memory");
+}
+__device__ __forceinline__ void rows_add(Mat<double> &st, const Rows &r, int odd) {
+  const Mat<double> m = rows_mat(r, odd);
+#pragma unroll
+  for (int k = 0; k < 9; k++) st.e[k / 3][k % 3] = cadd(st.e[k / 3][k % 3], m.e[k / 3][k % 3]);
 }
 
-// link (x, mu) from the FP64 12-real copy, row 2 rebuilt with the link's eta
-__device__ __forceinline__ Mat<double> link12_at(const double2 *U12, const LatticeDims &L, int x, int y, int z, int t,
-                                                 int mu) {
-  return load_link_d12(U12, L.Vh, mu, (x + y + z + t) & 1, half_index_i(L, x, y, z, t),
-                       eta_phase(L, x, y, z, t, mu));
+// number of phases (mod 2) of the link (c, MU); dt: c.t moved by that much
+template <int MU>
+__device__ __forceinline__ int phases(const LatticeDims &L, const SiteCoord &c, int dt = 0) {
+  if (MU == 0) return 0;
+  if (MU == 1) return c.x;
+  if (MU == 2) return c.x + c.y;
+  const int t = dt < 0 ? (c.t == 0 ? L.nt - 1 : c.t - 1) : c.t;
+  return c.x + c.y + c.z + (L.antiperiodic_t && t == L.nt - 1 ? 1 : 0);
+}
+
+// The staples of link (c, MU) in the plane with the N-th other direction,
+// added to st; la, lb hold the first two links (U_nu(x+mu), U_mu(x+nu)) on
+// entry and those of the next plane on return.  df, db: change of the half
+// index one step forward and backward (the index is a sum of one term per
+// coordinate, so two steps add up).
+template <int MU, int N>
+__device__ __forceinline__ void plane_loads(const double2 *U12, const LatticeDims &L, int par, int h,
+                                            const int (&df)[4], Rows &la, Rows &lb) {
+  constexpr int NU = N < MU ? N : N + 1;
+  rows_load(U12, L.Vh, NU, 1 - par, h + df[MU], la);
+  rows_load(U12, L.Vh, MU, 1 - par, h + df[NU], lb);
+}
+template <int MU, int N>
+__device__ __forceinline__ void plane_staples(const double2 *U12, const LatticeDims &L, int par, const SiteCoord &c,
+                                              int h, const int (&df)[4], const int (&db)[4], Rows &la, Rows &lb,
+                                              Mat<double> &st) {
+  constexpr int NU = N < MU ? N : N + 1;
+  const long Vh = L.Vh;
+  // phases: a step along d changes those of direction e > d
+  const int pn = phases<NU>(L, c), pm = phases<MU>(L, c);
+  const int n_at_mu = pn + (MU < NU), m_at_nu = pm + (NU < MU);  // U_nu(x+-mu), U_mu(x+-nu)
+  const int back = phases<NU>(L, c, -1);                         // U_nu(x-nu)
+  // upper: U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
+  Rows l3, a;
+  rows_load(U12, Vh, NU, par, h, l3);
+  a = rows_nd(la, rows_mat(lb, m_at_nu));
+  rows_fence(a);
+  Rows l4, l5;
+  rows_load(U12, Vh, NU, par, h + df[MU] + db[NU], l4);
+  rows_load(U12, Vh, MU, 1 - par, h + db[NU], l5);
+  a = rows_nd(a, rows_mat(l3, pn));
+  rows_add(st, a, n_at_mu + m_at_nu + pn);
+  mat_fence(st);
+  // lower: U_nu(x+mu-nu)^+ U_mu(x-nu)^+ U_nu(x-nu)
+  Rows l6;
+  rows_load(U12, Vh, NU, 1 - par, h + db[NU], l6);
+  const int n4 = back + (MU < NU);
+  {
+    const Mat<double> m = rows_mat(l4, n4);
+    Rows d;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int k = 0; k < 3; k++) d.e[i][k] = cconj(m.e[k][i]);
+    a = rows_nd(d, rows_mat(l5, m_at_nu));
+  }
+  rows_fence(a);
+  if constexpr (N < 2) plane_loads<MU, N + 1>(U12, L, par, h, df, la, lb);
+  else rows_load(U12, Vh, MU, par, h, la);  // U_mu(x) for the last product
+  a = rows_nn(a, rows_mat(l6, back));
+  rows_add(st, a, n4 + m_at_nu + back);
+  mat_fence(st);
+}
+
+template <int MU>
+__device__ __forceinline__ void gauge_force_link(const LatticeDims &L, const double2 *U12, double b3, double2 *ipdot,
+                                                 int accumulate, int par, int h) {
+  const long Vh = L.Vh;
+  const SiteCoord c = site_coords_i(L, par, h);
+  int df[4], db[4];
+#pragma unroll
+  for (int d = 0; d < 4; d++) {
+    df[d] = neighbour_i(L, c, d, +1) - h;
+    db[d] = neighbour_i(L, c, d, -1) - h;
+  }
+  Mat<double> st;
+#pragma unroll
+  for (int k = 0; k < 9; k++) st.e[k / 3][k % 3] = make_double2(0.0, 0.0);
+  Rows la, lb;
+  plane_loads<MU, 0>(U12, L, par, h, df, la, lb);
+  plane_staples<MU, 0>(U12, L, par, c, h, df, db, la, lb, st);
+  plane_staples<MU, 1>(U12, L, par, c, h, df, db, la, lb, st);
+  plane_staples<MU, 2>(U12, L, par, c, h, df, db, la, lb, st);
+  Mat<double> T = mmul(rows_mat(la, phases<MU>(L, c)), st);
+#pragma unroll
+  for (int k = 0; k < 9; k++) T.e[k / 3][k % 3] = cscale(T.e[k / 3][k % 3], b3);
+  T = ta(T);
+  if (accumulate) {
+    const Mat<double> old = load_aherm(ipdot, Vh, MU, par, h);
+#pragma unroll
+    for (int k = 0; k < 9; k++) T.e[k / 3][k % 3] = cadd(T.e[k / 3][k % 3], old.e[k / 3][k % 3]);
+  }
+  store_aherm(ipdot, Vh, MU, par, h, T);
 }
 
 // staples.cc:16-74 + ipdot.cc:25-79: ipdot_mu(x) = TA(U_mu(x) beta/3 sum_nu
 // [U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+ + U_nu(x+mu-nu)^+ U_mu(x-nu)^+ U_nu(x-nu)]).
-// Links from the FP64 12-real copy (96 instead of 144 bytes per load; each
-// thread loads 19), neighbours by compare-and-wrap in 32-bit arithmetic.
+// One link per lane, 19 link loads of 96 bytes, the links of each product
+// loaded during the product before it: 206 VGPRs, two waves per SIMD (three,
+// with 8 registers spilled, run the same).  32^3x8: 118 us per call (a form
+// that multiplied whole matrices and hoisted all loads, one wave per SIMD,
+// took 174); its FP64 multiply-adds alone are 42 us, its loads through L1
+// 49 us, its 168 MB 35 us.
 // Grid: the eight (parity, mu) workgroups of each kBlock-site tile
 // consecutive on one XCD, the tiles in the XCD-compact order of the Dslash
 // (tiles, or lattice order when null), so the links a tile's staples share
 // are fetched into that XCD's L2 together.
-__global__ __launch_bounds__(kBlock) void k_gauge_force(LatticeDims L, const int *tiles, const double2 *U12,
-                                                        double b3, double2 *ipdot, int accumulate) {
-  const long Vh = L.Vh;
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_gauge_force(
+    LatticeDims L, const int *tiles, const double2 *U12, double b3, double2 *ipdot, int accumulate) {
   const unsigned b = xcd_block(blockIdx.x, gridDim.x);
   const int mu = (int)(b & 3u);
   const int par = (int)((b >> 2) & 1u);
   const int q = (int)(b >> 3);
   const int h = (tiles ? tiles[q] : q) * kBlock + (int)threadIdx.x;
-  if (h >= (int)Vh) return;
-  const SiteCoord c = site_coords_i(L, par, h);
-  Mat<double> st;
-#pragma unroll
-  for (int i = 0; i < 3; i++)
-#pragma unroll
-    for (int k = 0; k < 3; k++) st.e[i][k] = make_double2(0.0, 0.0);
-  int x1 = c.x, y1 = c.y, z1 = c.z, t1 = c.t;  // x + mu
-  step_coord(L, x1, y1, z1, t1, mu, +1);
-  for (int nu = 0; nu < 4; nu++) {
-    if (nu == mu) continue;
-    // upper: U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
-    int x2 = c.x, y2 = c.y, z2 = c.z, t2 = c.t;
-    step_coord(L, x2, y2, z2, t2, nu, +1);
-    Mat<double> a = mmul_nd(link12_at(U12, L, x1, y1, z1, t1, nu), link12_at(U12, L, x2, y2, z2, t2, mu));
-    a = mmul_nd(a, link12_at(U12, L, c.x, c.y, c.z, c.t, nu));
-    // lower: U_nu(x+mu-nu)^+ U_mu(x-nu)^+ U_nu(x-nu)
-    int x3 = c.x, y3 = c.y, z3 = c.z, t3 = c.t;
-    step_coord(L, x3, y3, z3, t3, nu, -1);
-    int x4 = x1, y4 = y1, z4 = z1, t4 = t1;
-    step_coord(L, x4, y4, z4, t4, nu, -1);
-    const Mat<double> l1 = link12_at(U12, L, x4, y4, z4, t4, nu);
-    const Mat<double> l2 = link12_at(U12, L, x3, y3, z3, t3, mu);
-    Mat<double> b = mmul_dn(l1, mdag(l2));
-    b = mmul(b, link12_at(U12, L, x3, y3, z3, t3, nu));
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-      for (int k = 0; k < 3; k++) st.e[i][k] = cadd(st.e[i][k], cadd(a.e[i][k], b.e[i][k]));
+  if (h >= (int)L.Vh) return;
+  switch (mu) {
+    case 0: gauge_force_link<0>(L, U12, b3, ipdot, accumulate, par, h); break;
+    case 1: gauge_force_link<1>(L, U12, b3, ipdot, accumulate, par, h); break;
+    case 2: gauge_force_link<2>(L, U12, b3, ipdot, accumulate, par, h); break;
+    default: gauge_force_link<3>(L, U12, b3, ipdot, accumulate, par, h); break;
   }
-  const Mat<double> Um = link12_at(U12, L, c.x, c.y, c.z, c.t, mu);
-  Mat<double> T = mmul(Um, st);
-#pragma unroll
-  for (int i = 0; i < 3; i++)
-#pragma unroll
-    for (int k = 0; k < 3; k++) T.e[i][k] = cscale(T.e[i][k], b3);
-  T = ta(T);
-  if (accumulate) {
-    const Mat<double> old = load_aherm(ipdot, Vh, mu, par, h);
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-      for (int k = 0; k < 3; k++) T.e[i][k] = cadd(T.e[i][k], old.e[i][k]);
-  }
-  store_aherm(ipdot, Vh, mu, par, h, T);
 }
 
 int gauge_force(Context &c, int accumulate) {

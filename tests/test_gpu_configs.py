@@ -823,3 +823,28 @@ def test_host_transfers_round_trip(dims):
     for t in th:
         t.join()
     assert not err, err
+
+
+# ------------------------------------------------------------- gauge force
+@pytest.mark.parametrize("dims,antiperiodic", [((2, 2, 2, 2), True), ((2, 4, 6, 8), True), ((8, 2, 4, 2), False),
+                                               ((6, 6, 6, 6), True), ((16, 16, 16, 8), True), ((10, 8, 6, 4), False)])
+def test_gauge_force_against_oracle(dims, antiperiodic):
+    """The gauge force on extents of 2 (forward and backward neighbours
+    coincide), partly filled and permuted tiles and both temporal boundary
+    conditions, alone and added to a force: against the oracle's to 1e-13 (a
+    staple is three rounded products of unitary matrices, 1e-15)."""
+    lat = fields.Lattice(*dims, antiperiodic_t=antiperiodic)
+    U = fields.random_links(lat, 71, None)
+    F = 1j * fields.gauss_momenta(lat, 72)
+    say("gauge force", dims, antiperiodic)
+    g = Gpu(dims, mass=0.1, beta=5.7, antiperiodic_t=antiperiodic)
+    g.init0(U)
+    g.init1(ipdot=F)
+    ref = Oracle(dims, antiperiodic).ipdot_total(U, 5.7)
+    g.gauge_deriv(accumulate=True)
+    added = g.end(links=False, momenta=False)[1] - F
+    g.gauge_deriv()
+    alone = g.end(links=False, momenta=False)[1]
+    g.close()
+    assert rel(alone, ref) < 1e-13
+    assert rel(added, ref) < 1e-13
