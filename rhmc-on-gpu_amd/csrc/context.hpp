@@ -56,6 +56,7 @@ struct Context {
   float4 *U32 = nullptr;        // FP32 12-real copy, refreshed with U64
   double2 *U64c = nullptr;      // FP64 12-real copy, refreshed with U64
   double2 *U64_save = nullptr;  // Metropolis backup
+  bool links_stale = false;     // U64 and U32 behind U64c (inside an MD only)
   // algebra fields (8 reals/link)
   double2 *P = nullptr;      // momenta (hermitian)
   double2 *ipdot = nullptr;  // force (anti-hermitian)
@@ -179,7 +180,14 @@ int fermion_force_noalloc(Context &c, int order, const double *num, int accumula
 // fixed scratch (kept per device ordinal); sets c.noalloc_scratch
 int noalloc_scratch_init(Context &c);
 int gauge_force(Context &c, int accumulate);
-int exp_update(Context &c, double step);
+// gauge_force and momenta_update(step) in one pass
+int gauge_kick(Context &c, int accumulate, double step);
+// Link update.  keep: the copies brought up to date -- all, or inside an MD
+// those that it reads (the FP64 12-real one, with LINKS_FP32 the FP32 one
+// too); links_complete restores the others from the FP64 12-real copy.
+enum LinkCopies { LINKS_12 = 0, LINKS_FP32, LINKS_ALL };
+int exp_update(Context &c, double step, int keep = LINKS_ALL);
+int links_complete(Context &c);
 int momenta_update(Context &c, double step);
 // P <- s P
 int momenta_scale(Context &c, double s);

@@ -89,6 +89,8 @@ __device__ __forceinline__ void ff_systems(const C *own_v, const C *nb_v, long V
 // tile read as their own, and the +mu neighbours stay in the XCD's share, so
 // more of a spinor's five uses find it in that XCD's L2 (FP64, 128 systems
 // at 32^3x8: 5.84 -> 4.36 GB fetched per call, 816 -> 648 us).
+// U: the FP64 18-real links for FP64 solutions, the FP64 12-real copy for FP32
+// ones (the links an MD with FP32 solves keeps).
 template <typename C>
 __global__ __launch_bounds__(kBlock) void k_fermion_force(LatticeDims L, const int *tiles, const double2 *U,
                                                           const C *s, const C *hv, const double *coef, int nsys,
@@ -117,7 +119,9 @@ __global__ __launch_bounds__(kBlock) void k_fermion_force(LatticeDims L, const i
   for (int j = 0; j < nsys; j++) ff_systems<C, 1>(own_v, nb_v, Vh, j, ho, nbo, coef, sgn, F);
 #pragma unroll
   for (int mu = 0; mu < 4; mu++) {
-    const Mat<double> Um = load_link_d18(U, Vh, mu, par, h);
+    Mat<double> Um;
+    if constexpr (sizeof(C) == sizeof(double2)) Um = load_link_d18(U, Vh, mu, par, h);
+    else Um = load_link_d12(U, Vh, mu, par, h, eta_phase(L, c.x, c.y, c.z, c.t, mu));
     Mat<double> T = ta(mmul(Um, F[mu]));
     if (accumulate) {
       const Mat<double> old = load_aherm(ipdot, Vh, mu, par, h);
@@ -168,7 +172,7 @@ int fermion_force32(Context &c, int nsys, const double *num, const float2 *x32, 
   if (!hv || !coef || nsys > 256) return -1;
   if (!force_coef_upload(c, coef, num, nsys)) return -1;
   launch_hop_s(c, 1, x32, hv, nsys, 3 * Vh, 3 * Vh);
-  hipLaunchKernelGGL(k_fermion_force<float2>, dim3(2 * nblk(Vh)), dim3(kBlock), 0, c.stream, c.L, c.tiles, c.U64, x32, hv, coef,
+  hipLaunchKernelGGL(k_fermion_force<float2>, dim3(2 * nblk(Vh)), dim3(kBlock), 0, c.stream, c.L, c.tiles, c.U64c, x32, hv, coef,
                      nsys, c.ipdot, accumulate);
   // stream-ordered for the caller (the coefficients are staged in pinned memory)
   return hip_ok(c, hipGetLastError(), "fermion force") ? 0 : -1;
@@ -318,6 +322,23 @@ __device__ __forceinline__ void rows_add(Mat<double> &st, const Rows &r, int odd
   for (int k = 0; k < 9; k++) st.e[k / 3][k % 3] = cadd(st.e[k / 3][k % 3], m.e[k / 3][k % 3]);
 }
 
+// P += i step F at one link (momenta.cc:82-115): the force it has just formed
+__device__ __forceinline__ void mom_add(double2 *P, long Vh, int mu, int par, int h, const Mat<double> &F, double s) {
+  double2 *b = P + (long)(mu * 2 + par) * 4 * Vh + h;
+  const double2 f[3] = {F.e[0][1], F.e[0][2], F.e[1][2]};
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    double2 p = b[(long)k * Vh];
+    p.x -= s * f[k].y;
+    p.y += s * f[k].x;
+    b[(long)k * Vh] = p;
+  }
+  double2 d = b[3 * Vh];
+  d.x -= s * F.e[0][0].y;
+  d.y -= s * F.e[1][1].y;
+  b[3 * Vh] = d;
+}
+
 // number of phases (mod 2) of the link (c, MU); dt: c.t moved by that much
 template <int MU>
 __device__ __forceinline__ int phases(const LatticeDims &L, const SiteCoord &c, int dt = 0) {
@@ -384,7 +405,7 @@ __device__ __forceinline__ void plane_staples(const double2 *U12, const LatticeD
 
 template <int MU>
 __device__ __forceinline__ void gauge_force_link(const LatticeDims &L, const double2 *U12, double b3, double2 *ipdot,
-                                                 int accumulate, int par, int h) {
+                                                 int accumulate, double2 *P, double step, int par, int h) {
   const long Vh = L.Vh;
   const SiteCoord c = site_coords_i(L, par, h);
   int df[4], db[4];
@@ -411,6 +432,7 @@ __device__ __forceinline__ void gauge_force_link(const LatticeDims &L, const dou
     for (int k = 0; k < 9; k++) T.e[k / 3][k % 3] = cadd(T.e[k / 3][k % 3], old.e[k / 3][k % 3]);
   }
   store_aherm(ipdot, Vh, MU, par, h, T);
+  if (P) mom_add(P, Vh, MU, par, h, T, step);
 }
 
 // staples.cc:16-74 + ipdot.cc:25-79: ipdot_mu(x) = TA(U_mu(x) beta/3 sum_nu
@@ -426,7 +448,8 @@ __device__ __forceinline__ void gauge_force_link(const LatticeDims &L, const dou
 // (tiles, or lattice order when null), so the links a tile's staples share
 // are fetched into that XCD's L2 together.
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_gauge_force(
-    LatticeDims L, const int *tiles, const double2 *U12, double b3, double2 *ipdot, int accumulate) {
+    LatticeDims L, const int *tiles, const double2 *U12, double b3, double2 *ipdot, int accumulate, double2 *P,
+    double step) {
   const unsigned b = xcd_block(blockIdx.x, gridDim.x);
   const int mu = (int)(b & 3u);
   const int par = (int)((b >> 2) & 1u);
@@ -434,25 +457,35 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
   const int h = (tiles ? tiles[q] : q) * kBlock + (int)threadIdx.x;
   if (h >= (int)L.Vh) return;
   switch (mu) {
-    case 0: gauge_force_link<0>(L, U12, b3, ipdot, accumulate, par, h); break;
-    case 1: gauge_force_link<1>(L, U12, b3, ipdot, accumulate, par, h); break;
-    case 2: gauge_force_link<2>(L, U12, b3, ipdot, accumulate, par, h); break;
-    default: gauge_force_link<3>(L, U12, b3, ipdot, accumulate, par, h); break;
+    case 0: gauge_force_link<0>(L, U12, b3, ipdot, accumulate, P, step, par, h); break;
+    case 1: gauge_force_link<1>(L, U12, b3, ipdot, accumulate, P, step, par, h); break;
+    case 2: gauge_force_link<2>(L, U12, b3, ipdot, accumulate, P, step, par, h); break;
+    default: gauge_force_link<3>(L, U12, b3, ipdot, accumulate, P, step, par, h); break;
   }
 }
 
 int gauge_force(Context &c, int accumulate) {
   hipLaunchKernelGGL(k_gauge_force, dim3(8 * nblk(c.Vh)), dim3(kBlock), 0, c.stream, c.L, c.tiles, c.U64c,
-                     c.beta / 3.0, c.ipdot, accumulate);
+                     c.beta / 3.0, c.ipdot, accumulate, (double2 *)nullptr, 0.0);
   return hip_ok(c, hipGetLastError(), "gauge force") ? 0 : -1;
+}
+
+// the gauge force and the momentum update with it (gauge_force, then
+// momenta_update) in one pass
+int gauge_kick(Context &c, int accumulate, double step) {
+  hipLaunchKernelGGL(k_gauge_force, dim3(8 * nblk(c.Vh)), dim3(kBlock), 0, c.stream, c.L, c.tiles, c.U64c,
+                     c.beta / 3.0, c.ipdot, accumulate, c.P, step);
+  return hip_ok(c, hipGetLastError(), "gauge kick") ? 0 : -1;
 }
 
 // ------------------------------------------------------------ link update
 // momenta.cc:42-78 + su3.cc:187-219 + conf.cc:235-251:
 //   U <- Pi_SU3[ exp6(i step P) ] U, then Gram-Schmidt and row 2 *= eta.
-// Also refreshes the FP32 12-real copy used by the mixed-precision Dslash.
-__global__ __launch_bounds__(kBlock) void k_exp_update(LatticeDims L, const double2 *P, double step, double2 *U,
-                                                       float4 *U32, double2 *U64c) {
+// Writes the FP64 12-real copy and, when given, the 18-real links and the
+// FP32 copy; reads the 18-real links, or the 12-real copy when they are stale
+// (from12).
+__global__ __launch_bounds__(kBlock) void k_exp_update(LatticeDims L, const double2 *P, double step, const double2 *Uin,
+                                                       int from12, double2 *U, float4 *U32, double2 *U64c) {
   const long Vh = L.Vh;
   const int bx = xcd_block(blockIdx.x, gridDim.x);
   const long h = (long)bx * kBlock + threadIdx.x;
@@ -485,21 +518,47 @@ __global__ __launch_bounds__(kBlock) void k_exp_update(LatticeDims L, const doub
       for (int k = 0; k < 3; k++) E.e[i][k] = cadd(E.e[i][k], A.e[i][k]);
   }
   sunitarize(E);
-  Mat<double> Un = mmul(E, load_link_d18(U, Vh, mu, par, h));
-  sunitarize(Un);
-  const SiteCoord c = site_coords(L, par, h);
+  const SiteCoord c = site_coords_i(L, par, (int)h);
   const double eta = eta_phase(L, c.x, c.y, c.z, c.t, mu);
+  Mat<double> Un = mmul(E, from12 ? load_link_d12(Uin, Vh, mu, par, h, eta) : load_link_d18(Uin, Vh, mu, par, h));
+  sunitarize(Un);
 #pragma unroll
   for (int k = 0; k < 3; k++) Un.e[2][k] = cscale(Un.e[2][k], eta);
-  store_link_d18(U, Vh, mu, par, h, Un);
-  store_link_s12(U32, Vh, mu, par, h, Un);
+  if (U) store_link_d18(U, Vh, mu, par, h, Un);
+  if (U32) store_link_s12(U32, Vh, mu, par, h, Un);
   store_link_d12(U64c, Vh, mu, par, h, Un);
 }
 
-int exp_update(Context &c, double step) {
-  hipLaunchKernelGGL(k_exp_update, dim3(nblk(c.Vh), 2, 4), dim3(kBlock), 0, c.stream, c.L, c.P, step, c.U64, c.U32,
-                     c.U64c);
+// 18-real links and FP32 copy of the FP64 12-real copy
+__global__ __launch_bounds__(kBlock) void k_links_from12(LatticeDims L, const double2 *U64c, double2 *U, float4 *U32) {
+  const long Vh = L.Vh;
+  const long h = (long)blockIdx.x * kBlock + threadIdx.x;
+  const int par = blockIdx.y, mu = blockIdx.z;
+  if (h >= Vh) return;
+  const SiteCoord c = site_coords_i(L, par, (int)h);
+  const Mat<double> m = load_link_d12(U64c, Vh, mu, par, h, eta_phase(L, c.x, c.y, c.z, c.t, mu));
+  store_link_d18(U, Vh, mu, par, h, m);
+  store_link_s12(U32, Vh, mu, par, h, m);
+}
+
+// Inside an MD (keep below LINKS_ALL) only the copies its solves and forces
+// read are written: 256 bytes per link instead of 496 for a quenched one (32^3x8:
+// 85 -> 50 us per update), 304 with FP32 solves; links_complete then restores
+// the others, once.
+int exp_update(Context &c, double step, int keep) {
+  const bool all = keep == LINKS_ALL;
+  hipLaunchKernelGGL(k_exp_update, dim3(nblk(c.Vh), 2, 4), dim3(kBlock), 0, c.stream, c.L, c.P, step,
+                     c.links_stale ? c.U64c : c.U64, c.links_stale ? 1 : 0, all ? c.U64 : nullptr,
+                     keep >= LINKS_FP32 ? c.U32 : nullptr, c.U64c);
+  c.links_stale = !all;
   return hip_ok(c, hipGetLastError(), "exp update") ? 0 : -1;
+}
+
+int links_complete(Context &c) {
+  if (!c.links_stale) return 0;
+  c.links_stale = false;
+  hipLaunchKernelGGL(k_links_from12, dim3(nblk(c.Vh), 2, 4), dim3(kBlock), 0, c.stream, c.L, c.U64c, c.U64, c.U32);
+  return hip_ok(c, hipGetLastError(), "links complete") ? 0 : -1;
 }
 
 __global__ __launch_bounds__(kBlock) void k_refresh32(LatticeDims L, const double2 *U, float4 *U32, double2 *U64c) {

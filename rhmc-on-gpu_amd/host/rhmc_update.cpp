@@ -205,8 +205,9 @@ struct Traj {
     t_solve += secs(t0);
   }
 
-  // ipdot from the fermion force (+ gauge force when with_gauge)
-  void force(bool fermion, bool gauge) {
+  // ipdot from the fermion force (+ gauge force when with_gauge, whose pass
+  // also updates the momenta by step)
+  void force(bool fermion, bool gauge, double step) {
     const int n = (int)L.size();
     if (fermion && !p.pure_gauge) {
       const bool f32 = L[0].md_fp32();
@@ -228,24 +229,27 @@ struct Traj {
         const int rcf = f32 ? fermion_force32(c, c.n_pf * order, coef.data(), c.smf32, 0)
                             : fermion_force(c, c.n_pf * order, coef.data(), c.smf, 0);
         if (rcf) la.fail(-1);
-        if (gauge) gauge_force(c, 1);
+        if (gauge) gauge_kick(c, 1, step);
       }
       mark(ev_force);
     } else {
       mark(ev_force);
-      for (Lat &la : L) gauge_force(la.c, 0);
+      for (Lat &la : L) gauge_kick(la.c, 0, step);
       mark(ev_force);
     }
   }
+  // the link copies the MD reads between its updates
+  int md_links() const { return p.pure_gauge ? LINKS_12 : L[0].md_fp32() ? LINKS_FP32 : LINKS_ALL; }
   void P(double step, bool fermion, bool gauge) {
-    force(fermion, gauge);
+    force(fermion, gauge, step);
+    if (gauge || !fermion || p.pure_gauge || !ok()) return;  // momenta updated with the gauge force
     mark(ev_update);
     for (Lat &la : L) momenta_update(la.c, step);
     mark(ev_update);
   }
   void Q(double step) {
     mark(ev_update);
-    for (Lat &la : L) exp_update(la.c, step);
+    for (Lat &la : L) exp_update(la.c, step, md_links());
     mark(ev_update);
   }
 
@@ -349,6 +353,8 @@ struct Traj {
     else if (p.integrator == RHMC_INT_MULTISTEP_2MN) ms2mn();
     else if (p.integrator == RHMC_INT_MULTISTEP_4MN) ms4mn();
     else leapfrog();
+    for (Lat &la : L)
+      if (links_complete(la.c)) la.fail(-1);
   }
 };
 
