@@ -227,8 +227,8 @@ int kernel_timing_stamps(Context &c, size_t n);
 
 // persistent workspace buffers of the gauge-field kernels (grown on demand,
 // freed with the context): the force's hop outputs and coefficients, the
-// rational sums' coefficients
-enum ScratchUse { SCR_FORCE_HOP = 0, SCR_FORCE_COEF, SCR_SOLSUM_COEF, SCR_COUNT };
+// rational sums' coefficients, the measurements' fields, sums
+enum ScratchUse { SCR_FORCE_HOP = 0, SCR_FORCE_COEF, SCR_SOLSUM_COEF, SCR_MEAS, SCR_SUMS, SCR_COUNT };
 void *scratch_get(Context &c, int use, size_t bytes);
 // small host <-> device transfers through pinned staging (pageable copies
 // cost a runtime staging pass with the GPU idle): h2d is enqueued on

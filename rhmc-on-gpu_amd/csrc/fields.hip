@@ -20,19 +20,6 @@ namespace rhmc {
 
 static inline unsigned nblk(long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
-__device__ __forceinline__ Mat<double> link_at(const double2 *U, const LatticeDims &L, int x, int y, int z, int t,
-                                               int mu) {
-  const int par = (x + y + z + t) & 1;
-  return load_link_d18(U, L.Vh, mu, par, half_index(L, x, y, z, t));
-}
-
-__device__ __forceinline__ void shift_coord(const LatticeDims &L, int &x, int &y, int &z, int &t, int mu, int d) {
-  if (mu == 0) x = (x + d + L.nx) % L.nx;
-  else if (mu == 1) y = (y + d + L.ny) % L.ny;
-  else if (mu == 2) z = (z + d + L.nz) % L.nz;
-  else t = (t + d + L.nt) % L.nt;
-}
-
 // --------------------------------------------------------------- fermion force
 // fermionforce.cc:46-104 + ipdot.cc:83-155:
 //   F_mu(e) =  sum_j a_j h_j(e+mu) (x) s_j(e)^*     (even sites)
@@ -644,32 +631,47 @@ int sol_sum(Context &c, double2 *io, const double2 *x, int nshift, double a0, co
 }
 
 // ------------------------------------------------------------------- action
+// Re tr of the plaquette (x; mu, nu) from the 18-real links: with A = U_mu(x)
+// U_nu(x+mu) and B = U_nu(x) U_mu(x+nu) it is the real part of sum A_ij B_ij^*, two
+// matrix products and nine complex ones instead of three products.  mu and
+// nu are the same in a wave; one copy of the code for all planes (a kernel
+// that runs once per measurement mostly waits for its instructions).
+__device__ __forceinline__ double plaq_re(const LatticeDims &L, const double2 *U, int par, int h, const SiteCoord &c,
+                                          int mu, int nu) {
+  const long Vh = L.Vh;
+  const int hm = neighbour_i(L, c, mu, +1), hn = neighbour_i(L, c, nu, +1);
+  const Mat<double> a = mmul(load_link_d18(U, Vh, mu, par, h), load_link_d18(U, Vh, nu, 1 - par, hm));
+  const Mat<double> b = mmul(load_link_d18(U, Vh, nu, par, h), load_link_d18(U, Vh, mu, 1 - par, hn));
+  double s = 0.0;
+#pragma unroll
+  for (int k = 0; k < 9; k++) {
+    s = fmar(a.e[k / 3][k % 3].x, b.e[k / 3][k % 3].x, s);
+    s = fmar(a.e[k / 3][k % 3].y, b.e[k / 3][k % 3].y, s);
+  }
+  return s;
+}
+
 // action.cc:6-156: per-site contributions in the reference's order
 //   init 0 : v  = sum_plaq beta/3 Re tr(plaq) + sum_mu 1/2 Re tr P^2 + sum_ps |phi|^2
 //   init -1: v -= the same with Re<phi_new, chi> for the fermions
 __global__ __launch_bounds__(kBlock) void k_action(LatticeDims L, const double2 *U, const double2 *P, double b3,
                                                    const double2 *phi, const double2 *chi, int npf, int with_f,
                                                    double *value, int init) {
+  // both parities of a tile follow each other on one XCD, each XCD a part of
+  // the lattice (32^3x8: 117 -> 89 us)
   const long Vh = L.Vh;
-  const long h = (long)blockIdx.x * kBlock + threadIdx.x;
-  const int par = blockIdx.y;
+  const unsigned b = xcd_block(blockIdx.x, gridDim.x);
+  const int par = (int)(b & 1u);
+  const long h = (long)(b >> 1) * kBlock + threadIdx.x;
   if (h >= Vh) return;
   const long idx = (long)par * Vh + h;
-  const SiteCoord c = site_coords(L, par, h);
   double v = init == 0 ? 0.0 : value[idx];
   const double sg = init == 0 ? 1.0 : -1.0;
+  const SiteCoord c = site_coords_i(L, par, (int)h);
+#pragma unroll 1
   for (int mu = 0; mu < 3; mu++)
-    for (int nu = mu + 1; nu < 4; nu++) {
-      int x1 = c.x, y1 = c.y, z1 = c.z, t1 = c.t;
-      shift_coord(L, x1, y1, z1, t1, mu, +1);
-      int x2 = c.x, y2 = c.y, z2 = c.z, t2 = c.t;
-      shift_coord(L, x2, y2, z2, t2, nu, +1);
-      Mat<double> a = mmul(load_link_d18(U, Vh, mu, par, h), link_at(U, L, x1, y1, z1, t1, nu));
-      a = mmul_nd(a, link_at(U, L, x2, y2, z2, t2, mu));
-      a = mmul_nd(a, load_link_d18(U, Vh, nu, par, h));
-      const double p = b3 * (a.e[0][0].x + a.e[1][1].x + a.e[2][2].x);
-      v += sg * p;
-    }
+#pragma unroll 1
+    for (int nu = mu + 1; nu < 4; nu++) v += sg * b3 * plaq_re(L, U, par, (int)h, c, mu, nu);
   for (int mu = 0; mu < 4; mu++) {
     const Mat<double> pm = load_herm(P, Vh, mu, par, h);
     const Mat<double> q = mmul(pm, pm);
@@ -690,73 +692,114 @@ __global__ __launch_bounds__(kBlock) void k_action(LatticeDims L, const double2 
 }
 
 int action_local(Context &c, const double2 *phi, const double2 *chi, int with_f, int init) {
-  hipLaunchKernelGGL(k_action, dim3(nblk(c.Vh), 2), dim3(kBlock), 0, c.stream, c.L, c.U64, c.P, c.beta / 3.0, phi,
+  hipLaunchKernelGGL(k_action, dim3(2 * nblk(c.Vh)), dim3(kBlock), 0, c.stream, c.L, c.U64, c.P, c.beta / 3.0, phi,
                      chi, c.n_pf, with_f, c.action, init);
   return hip_ok(c, hipGetLastError(), "action") ? 0 : -1;
 }
 
-// include/tools.h:25-57 pairwise fold, same association order as the reference
-__global__ __launch_bounds__(kBlock) void k_fold(double *v, long j, long off) {
+// include/tools.h:25-57 pairwise fold, same association order as the
+// reference: n even, v[k] += v[k + n/2] for k < n/2; n odd, v[k] += v[k + n/2
+// + 1] for k < n/2 and the middle value stays.  Array y of a launch starts at
+// v + y stride.
+__global__ __launch_bounds__(kBlock) void k_fold(double *v, long stride, long j, long off) {
   const long k = (long)blockIdx.x * kBlock + threadIdx.x;
+  v += blockIdx.y * stride;
   if (k < j) v[k] += v[k + off];
 }
-
-// the reference's pairwise tree sum (include/tools.h:25-57) of v[0..n), in place
-static void pairwise_sum(Context &c, double *v, long n) {
+// LV halvings at once: value k of n / 2^LV gathers the 2^LV values that the
+// halvings add to it, in their order
+template <int LV>
+__global__ __launch_bounds__(kBlock) void k_fold_levels(double *v, long stride, long m) {
+  const long k = (long)blockIdx.x * kBlock + threadIdx.x;
+  v += blockIdx.y * stride;
+  if (k >= m) return;
+  double a[1 << LV];
+#pragma unroll
+  for (int i = 0; i < 1 << LV; i++) a[i] = v[k + i * m];
+#pragma unroll
+  for (int w = 1 << (LV - 1); w > 0; w /= 2)
+#pragma unroll
+    for (int i = 0; i < w; i++) a[i] += a[i + w];
+  v[k] = a[0];
+}
+// the remaining levels of up to kFoldLast values, in workgroup memory; array
+// y's sum to out[y]
+constexpr int kFoldLast = 4096;
+__global__ __launch_bounds__(1024) void k_fold_last(const double *v, long stride, int n, double *out) {
+  __shared__ double s[kFoldLast];
+  v += blockIdx.x * stride;
+  for (int k = threadIdx.x; k < n; k += 1024) s[k] = v[k];
+  __syncthreads();
   while (n > 1) {
-    long j, off, next;
-    if (n % 2 == 0) { j = n / 2; off = j; next = j; }
-    else { j = n / 2; off = j + 1; next = j + 1; }
-    hipLaunchKernelGGL(k_fold, dim3(nblk(j)), dim3(kBlock), 0, c.stream, v, j, off);
-    n = next;
+    const int j = n / 2, off = n - j;
+    for (int k = threadIdx.x; k < j; k += 1024) s[k] += s[k + off];
+    __syncthreads();
+    n = off;
   }
+  if (threadIdx.x == 0) out[blockIdx.x] = s[0];
+}
+
+// The reference's pairwise tree sums of `arrays` arrays of n values (stride
+// apart; overwritten) into out[arrays] on the device: two or three launches
+// instead of one per level (18 for 2^18 values, 3 us each).
+static void pairwise_sums(Context &c, double *v, long n, long stride, int arrays, double *out) {
+  while (n > kFoldLast) {
+    const int lv = n % 32 == 0 ? 5 : n % 8 == 0 ? 3 : n % 2 == 0 ? 1 : 0;
+    const long m = lv ? n >> lv : n / 2;
+    const dim3 grid(nblk(m), (unsigned)arrays);
+    if (lv == 5) hipLaunchKernelGGL(k_fold_levels<5>, grid, dim3(kBlock), 0, c.stream, v, stride, m);
+    else if (lv == 3) hipLaunchKernelGGL(k_fold_levels<3>, grid, dim3(kBlock), 0, c.stream, v, stride, m);
+    else if (lv == 1) hipLaunchKernelGGL(k_fold_levels<1>, grid, dim3(kBlock), 0, c.stream, v, stride, m);
+    else hipLaunchKernelGGL(k_fold, grid, dim3(kBlock), 0, c.stream, v, stride, m, n - m);
+    n = lv ? m : n - m;
+  }
+  hipLaunchKernelGGL(k_fold_last, dim3((unsigned)arrays), dim3(1024), 0, c.stream, v, stride, (int)n, out);
 }
 
 int action_sum(Context &c, double *out) {
-  pairwise_sum(c, c.action, c.V);
-  return d2h_sync(c, out, c.action, sizeof(double)) ? 0 : -1;
+  double *sum = (double *)scratch_get(c, SCR_SUMS, sizeof(double));
+  if (!sum) return -1;
+  pairwise_sums(c, c.action, c.V, c.V, 1, sum);
+  return d2h_sync(c, out, sum, sizeof(double)) ? 0 : -1;
 }
 
 // ------------------------------------------------------------ measurements
 // gaugemeas.cc:6-66 (Conf::calc_plaq): per site minus Re tr of its three
-// temporal (nu = 3) and three spatial plaquettes, at the reference site index
-__global__ __launch_bounds__(kBlock) void k_plaq(LatticeDims L, const double2 *U, double *vt, double *vs) {
-  const long Vh = L.Vh;
-  const long h = (long)blockIdx.x * kBlock + threadIdx.x;
-  const int par = blockIdx.y;
-  if (h >= Vh) return;
-  const SiteCoord c = site_coords(L, par, h);
-  double st = 0.0, ss = 0.0;
-  for (int mu = 0; mu < 3; mu++)
-    for (int nu = mu + 1; nu < 4; nu++) {
-      int x1 = c.x, y1 = c.y, z1 = c.z, t1 = c.t;
-      shift_coord(L, x1, y1, z1, t1, mu, +1);
-      int x2 = c.x, y2 = c.y, z2 = c.z, t2 = c.t;
-      shift_coord(L, x2, y2, z2, t2, nu, +1);
-      Mat<double> a = mmul(link_at(U, L, c.x, c.y, c.z, c.t, mu), link_at(U, L, x1, y1, z1, t1, nu));
-      a = mmul_nd(a, link_at(U, L, x2, y2, z2, t2, mu));
-      a = mmul_nd(a, link_at(U, L, c.x, c.y, c.z, c.t, nu));
-      const double re = a.e[0][0].x + a.e[1][1].x + a.e[2][2].x;
-      if (nu == 3) st -= re;
-      else ss -= re;
-    }
-  const long idx = (long)par * Vh + h;
-  vt[idx] = st;
-  vs[idx] = ss;
+// temporal (nu = 3) and three spatial plaquettes, at the reference site
+// index.  A workgroup takes 64 sites, a wave per plane; a tile's four
+// workgroups (parity, temporal or spatial) follow each other on one XCD and
+// each XCD has a contiguous part of the lattice, so that the links the
+// plaquettes share come from its L2.  24^3x6: 17 us (a grid that spread
+// neighbouring tiles over the XCDs 28, one thread for all six planes 37).
+__global__ __launch_bounds__(192) void k_plaq(LatticeDims L, const double2 *U, double *vt, double *vs) {
+  __shared__ double sh[2][64];
+  const int lane = threadIdx.x & 63, plane = threadIdx.x >> 6;
+  const unsigned b = xcd_block(blockIdx.x, gridDim.x);
+  const int spatial = (int)(b & 1u), par = (int)((b >> 1) & 1u);
+  const int h = (int)(b >> 2) * 64 + lane;
+  const bool in = h < (int)L.Vh;
+  // planes (plane, 3), or (0, 1), (0, 2), (1, 2)
+  const int mu = __builtin_amdgcn_readfirstlane(spatial ? plane >> 1 : plane);
+  const int nu = __builtin_amdgcn_readfirstlane(spatial ? 1 + ((plane + 1) >> 1) : 3);
+  const double p = in ? plaq_re(L, U, par, h, site_coords_i(L, par, h), mu, nu) : 0.0;
+  if (plane) sh[plane - 1][lane] = p;
+  __syncthreads();
+  if (plane == 0 && in) (spatial ? vs : vt)[(long)par * L.Vh + h] = -p - sh[0][lane] - sh[1][lane];
 }
 
 // gaugemeas.cc:70-104 (Conf::calc_poly): one line per spatial point, from
 // the sites r < vol3 (even parity, t = 0 or 1), minus the trace
 __global__ __launch_bounds__(kBlock) void k_poly(LatticeDims L, const double2 *U, double *vre, double *vim,
                                                  long vol3) {
-  const long r = (long)blockIdx.x * kBlock + threadIdx.x;
+  const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= vol3) return;
-  const SiteCoord c = site_coords(L, 0, r);
-  Mat<double> a = link_at(U, L, c.x, c.y, c.z, c.t, 3);
-  int t = c.t;
+  const SiteCoord c = site_coords_i(L, 0, (int)r);
+  int t = c.t, par = 0;
+  Mat<double> a = load_link_d18(U, L.Vh, 3, 0, r);
   for (int k = 1; k < L.nt; k++) {
     t = t + 1 == L.nt ? 0 : t + 1;
-    a = mmul(a, link_at(U, L, c.x, c.y, c.z, t, 3));
+    par ^= 1;
+    a = mmul(a, load_link_d18(U, L.Vh, 3, par, half_index_i(L, c.x, c.y, c.z, t)));
   }
   vre[r] = -(a.e[0][0].x + a.e[1][1].x + a.e[2][2].x);
   vim[r] = -(a.e[0][0].y + a.e[1][1].y + a.e[2][2].y);
@@ -860,10 +903,9 @@ __global__ __launch_bounds__(kBlock) void k_chiral_terms(LatticeDims L, const do
 int chiral_meas(Context &c, const double *rnd_e_h, const double *rnd_o_h, unsigned long long seed, double res,
                 int max_cg, double n_flavours, double *out, int *iters) {
   const long Vh = c.Vh, n3 = 3 * Vh;
-  double2 *buf = nullptr;
-  double *w = nullptr;
-  if (!hip_ok(c, hipMallocAsync((void **)&buf, sizeof(double2) * n3 * 6, c.stream), "chiral")) return -1;
-  if (!hip_ok(c, hipMallocAsync((void **)&w, sizeof(double) * 8 * Vh, c.stream), "chiral")) return -1;
+  double2 *buf = (double2 *)scratch_get(c, SCR_MEAS, sizeof(double2) * n3 * 6 + sizeof(double) * (8 * Vh + 8));
+  if (!buf) return -1;
+  double *w = (double *)(buf + 6 * n3);
   double2 *re_ = buf, *ro = buf + n3, *phi = buf + 2 * n3, *ce = buf + 3 * n3, *co = buf + 4 * n3, *tmp = buf + 5 * n3;
   if (rnd_e_h && rnd_o_h) {
     if (upload_spinors(c, rnd_e_h, re_, 1) || upload_spinors(c, rnd_o_h, ro, 1)) return -1;
@@ -876,22 +918,14 @@ int chiral_meas(Context &c, const double *rnd_e_h, const double *rnd_o_h, unsign
   const double shift0 = 0.0;
   int it = 0;
   const int rc = multishift_solve(c, phi, 1, 1, &shift0, res, 0, PREC_FP64, max_cg, ce, &it);
-  if (rc) {
-    hipFreeAsync(buf, c.stream);
-    hipFreeAsync(w, c.stream);
-    hipStreamSynchronize(c.stream);
-    return rc;
-  }
+  if (rc) return rc;
   launch_hop_d(c, 1, ce, tmp, 1, n3, n3);  // D_oe chi_e
   const double im = 1.0 / c.mass;
   hipLaunchKernelGGL(k_axpby, dim3(nblk(n3)), dim3(kBlock), 0, c.stream, co, ro, tmp, im, -im, n3);
   hipLaunchKernelGGL(k_chiral_terms, dim3(nblk(Vh)), dim3(kBlock), 0, c.stream, c.L, c.U64, re_, ro, ce, co, w);
-  for (int k = 0; k < 8; k++) pairwise_sum(c, w + k * Vh, Vh);
+  pairwise_sums(c, w, Vh, Vh, 8, w + 8 * Vh);
   double h[8];
-  for (int k = 0; k < 8; k++) hipMemcpyAsync(&h[k], w + k * Vh, sizeof(double), hipMemcpyDeviceToHost, c.stream);
-  hipFreeAsync(buf, c.stream);
-  hipFreeAsync(w, c.stream);
-  if (!hip_ok(c, hipStreamSynchronize(c.stream), "chiral")) return -1;
+  if (!d2h_sync(c, h, w + 8 * Vh, sizeof(h))) return -1;
   const double inv_size = 1.0 / (double)c.V;
   const double f0 = n_flavours * 0.25 * inv_size, f1 = 0.5 * n_flavours * 0.25 * inv_size;
   out[0] = h[0] * f0; out[1] = h[1] * f0;
@@ -901,23 +935,16 @@ int chiral_meas(Context &c, const double *rnd_e_h, const double *rnd_o_h, unsign
 }
 
 int gauge_meas(Context &c, double *pls, double *plt, double *pre, double *pim) {
-  double *w = nullptr;
   const long vol3 = (long)c.L.nx * c.L.ny * c.L.nz;
-  if (!hip_ok(c, hipMallocAsync((void **)&w, sizeof(double) * (2 * c.V + 2 * vol3), c.stream), "meas")) return -1;
-  double *vt = w, *vs = w + c.V, *vre = w + 2 * c.V, *vim = vre + vol3;
-  hipLaunchKernelGGL(k_plaq, dim3(nblk(c.Vh), 2), dim3(kBlock), 0, c.stream, c.L, c.U64, vt, vs);
-  hipLaunchKernelGGL(k_poly, dim3(nblk(vol3)), dim3(kBlock), 0, c.stream, c.L, c.U64, vre, vim, vol3);
-  pairwise_sum(c, vt, c.V);
-  pairwise_sum(c, vs, c.V);
-  pairwise_sum(c, vre, vol3);
-  pairwise_sum(c, vim, vol3);
+  double *w = (double *)scratch_get(c, SCR_MEAS, sizeof(double) * (2 * c.V + 2 * vol3 + 4));
+  if (!w) return -1;
+  double *vt = w, *vs = w + c.V, *vre = w + 2 * c.V, *vim = vre + vol3, *sums = vim + vol3;
+  hipLaunchKernelGGL(k_plaq, dim3((unsigned)((c.Vh + 63) / 64 * 4)), dim3(192), 0, c.stream, c.L, c.U64, vt, vs);
+  hipLaunchKernelGGL(k_poly, dim3((unsigned)((vol3 + 63) / 64)), dim3(64), 0, c.stream, c.L, c.U64, vre, vim, vol3);
+  pairwise_sums(c, vt, c.V, c.V, 2, sums);
+  pairwise_sums(c, vre, vol3, vol3, 2, sums + 2);
   double h[4];
-  hipMemcpyAsync(&h[0], vt, sizeof(double), hipMemcpyDeviceToHost, c.stream);
-  hipMemcpyAsync(&h[1], vs, sizeof(double), hipMemcpyDeviceToHost, c.stream);
-  hipMemcpyAsync(&h[2], vre, sizeof(double), hipMemcpyDeviceToHost, c.stream);
-  hipMemcpyAsync(&h[3], vim, sizeof(double), hipMemcpyDeviceToHost, c.stream);
-  hipFreeAsync(w, c.stream);
-  if (!hip_ok(c, hipStreamSynchronize(c.stream), "meas")) return -1;
+  if (!d2h_sync(c, h, sums, sizeof(h))) return -1;
   // the reference's normalisation order: sum * (1/V/3.) * one_by_three
   const double inv_size_by_three = 1.0 / (double)c.V / 3.;
   const double inv_vol3 = 1.0 / (double)vol3;

@@ -50,7 +50,7 @@ enum Slot {
   S_PARTIAL2, S_BASIS, S_BSH, S_HIST, S_COEF, S_HPART,
   S_FORCE_H, S_FORCE_COEF, S_SOLSUM_COEF,
   S_RS_SRC, S_RS_Y, S_RS_IDX, S_GROUP_TAB,
-  S_RES_H, S_RES_PART,
+  S_RES_H, S_RES_PART, S_MEAS, S_ACTION_SUM,
   S_COUNT
 };
 
@@ -217,7 +217,7 @@ bool d2h_sync(Context &c, void *dst, const void *src, size_t bytes) {
 // workspace buffers of the gauge-field side (fields.hip), kept for the
 // context's lifetime instead of an allocation per MD force
 void *scratch_get(Context &c, int use, size_t bytes) {
-  static const int slot[SCR_COUNT] = {S_FORCE_H, S_FORCE_COEF, S_SOLSUM_COEF};
+  static const int slot[SCR_COUNT] = {S_FORCE_H, S_FORCE_COEF, S_SOLSUM_COEF, S_MEAS, S_ACTION_SUM};
   return use >= 0 && use < SCR_COUNT ? ws_get(c, slot[use], bytes) : nullptr;
 }
 

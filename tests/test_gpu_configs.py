@@ -848,3 +848,28 @@ def test_gauge_force_against_oracle(dims, antiperiodic):
     g.close()
     assert rel(alone, ref) < 1e-13
     assert rel(added, ref) < 1e-13
+
+
+# ------------------------------------------------- loops and pairwise sums
+@pytest.mark.parametrize("dims", [(2, 2, 2, 2), (4, 4, 4, 4), (6, 10, 4, 14), (14, 14, 14, 10), (18, 18, 18, 18),
+                                  (32, 16, 16, 16)])
+def test_loops_and_action_sums(dims):
+    """Plaquettes, Polyakov loop and the action over site counts that the
+    pairwise sums take by 5, 3 and 1 levels at a time, with an odd count above
+    the last launch's size (18^4) and below it: against the oracle's loops to
+    1e-13 and its action to 1e-12 of the sum of absolute values (each term is
+    rounded at 1e-15, the sums are in the same order)."""
+    lat = fields.Lattice(*dims)
+    U = fields.random_links(lat, 81, 0.3)
+    P = fields.gauss_momenta(lat, 82)
+    say("loops", dims)
+    o = Oracle(dims)
+    g = Gpu(dims, mass=0.1, beta=5.7)
+    g.init0(U)
+    g.init1(momenta=P)
+    for a, b in zip(g.gauge_meas(), o.gauge_meas(U)):
+        assert abs(a - b) < 1e-13
+    g.action(0, with_fermions=False)
+    v = o.action(U, P, 5.7, None, None, with_fermions=False)
+    assert abs(g.action_sum() - o.global_sum(v.copy())) < 1e-12 * np.abs(v).sum()
+    g.close()
