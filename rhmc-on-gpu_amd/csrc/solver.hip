@@ -1556,8 +1556,9 @@ static void dslash_launch(Context &c, DsArgs &a, int code) {
 // * for the reducing M^dag M launches, the tiles per workgroup (1, 2, 4:
 //   fewer, longer workgroups and fewer reduction partials).
 // On the first launch of each (precision, links, mode, reduction, nvec)
-// every candidate is timed in place with HIP events and the fastest is kept
-// for the lifetime of the context -- and, when a tuning cache file is set
+// the candidates are timed in place with HIP events, the clearly slower ones
+// once (all ten times each took 2.6 s of a first 48^3x12 trajectory), and the
+// fastest is kept for the lifetime of the context -- and, when a tuning cache file is set
 // (RHMC_TUNE_CACHE or gpu_tune_cache), stored there under (kernel, lattice
 // extents, precision, nvec, GPU architecture) and reused by later contexts
 // and processes without timing.  The launches are idempotent, except the
@@ -1566,6 +1567,8 @@ static void dslash_launch(Context &c, DsArgs &a, int code) {
 // launch write is overwritten by the final launch.  RHMC_DSLASH_NR ("4", "4x4" or "2t4")
 // forces the right-hand sides per lane, lanes per site and tiles per workgroup.
 constexpr int kTuneRounds = 3;
+constexpr float kTuneDrop = 1.5f, kTuneFirst = 0.2f;   // ms: a kernel's first launch
+constexpr float kTuneKeep = 1.2f, kTuneNoise = 0.004f; // ms: spread of single launches
 
 template <typename R, int LINK, int MODE, int RED>
 static void dslash_dispatch(Context &c, DsArgs &a) {
@@ -1603,21 +1606,36 @@ static void dslash_dispatch(Context &c, DsArgs &a) {
       for (int v = 1; v <= 8 && v <= std::max(1, a.nvec); v *= 2)
         for (int ident = c.tiles ? 0 : 1; ident <= 1; ident++)
           for (int tpw = 0; tpw <= (reducing ? 2 : 0); tpw++) cands.push_back(make_shape(v, lanes, ident, tpw));
-    // every candidate launched once, then the best of kTuneRounds interleaved
-    // rounds of 3 launches each (one round alone picked the FP32 8-RHS hop's
-    // shape differently from run to run: 26.2 or 28.6 us per launch)
-    for (const int cand : cands) dslash_launch<R, LINK, MODE, RED>(c, t, cand);
-    std::vector<float> cand_ms(cands.size(), 1e30f);
+    // every candidate launched once, dropped when that took kTuneDrop times
+    // the fastest so far (and a first launch's code loading) or more; of the
+    // others, once more, those within kTuneKeep of the fastest go on to the
+    // best of kTuneRounds interleaved rounds of 3 launches each (one round
+    // alone picked the FP32 8-RHS hop's shape differently from run to run:
+    // 26.2 or 28.6 us per launch)
+    auto timed = [&](int cand, int n) {
+      hipEventRecord(e0, c.stream);
+      for (int k = 0; k < n; k++) dslash_launch<R, LINK, MODE, RED>(c, t, cand);
+      hipEventRecord(e1, c.stream);
+      hipEventSynchronize(e1);
+      float ms = 0.f;
+      hipEventElapsedTime(&ms, e0, e1);
+      return ms;
+    };
+    auto keep = [&](const std::vector<float> &ms, float limit) {
+      std::vector<int> left;
+      for (size_t i = 0; i < cands.size(); i++)
+        if (ms[i] <= limit) left.push_back(cands[i]);
+      cands = left;
+    };
+    std::vector<float> cand_ms;
+    for (const int cand : cands) cand_ms.push_back(timed(cand, 1));
+    keep(cand_ms, kTuneDrop * *std::min_element(cand_ms.begin(), cand_ms.end()) + kTuneFirst);
+    cand_ms.clear();
+    for (const int cand : cands) cand_ms.push_back(timed(cand, 1));
+    keep(cand_ms, kTuneKeep * *std::min_element(cand_ms.begin(), cand_ms.end()) + kTuneNoise);
+    cand_ms.assign(cands.size(), 1e30f);
     for (int round = 0; round < kTuneRounds; round++)
-      for (size_t i = 0; i < cands.size(); i++) {
-        hipEventRecord(e0, c.stream);
-        for (int k = 0; k < 3; k++) dslash_launch<R, LINK, MODE, RED>(c, t, cands[i]);
-        hipEventRecord(e1, c.stream);
-        hipEventSynchronize(e1);
-        float ms = 0.f;
-        hipEventElapsedTime(&ms, e0, e1);
-        cand_ms[i] = std::min(cand_ms[i], ms);
-      }
+      for (size_t i = 0; i < cands.size(); i++) cand_ms[i] = std::min(cand_ms[i], timed(cands[i], 3));
     for (size_t i = 0; i < cands.size(); i++)
       if (cand_ms[i] < best) {
         best = cand_ms[i];
