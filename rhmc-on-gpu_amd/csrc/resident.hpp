@@ -49,7 +49,7 @@ struct ResArgs {
   const void *U;
   void *basis, *h;       // slots of stride elements: r^(k) at slot k, h of iteration k at slot k-1
   long stride;           // right-hand sides of the whole solve * 3 * Vh
-  double diag;           // m^2
+  const double *diag;    // per system m^2 + its shift
   const BmsShared *sh;   // rho_0 and the zero-source stops of the set-up
   MsState *ms;
   BmsHist *hist;
@@ -106,7 +106,7 @@ __device__ __forceinline__ double wave_sum_dpp(double v) {
 template <int NR>
 struct ResShared {
   double wave[2][kResMaxWaves][NR];  // wave sums: own partial, all partials
-  double rho1[NR], rho2[NR], beta[NR], alpha[NR];
+  double diag[NR], rho1[NR], rho2[NR], beta[NR], alpha[NR];
   double coef[2][NR];                // alpha and c of the residual update
   int stop[NR], next[NR];            // stopped before this / the next iteration
   int aborted;
@@ -301,6 +301,9 @@ __device__ __forceinline__ void res_body(const ResArgs &a, int wg, int copy, lon
   bool mine[P];
   unsigned own[P];  // element of this lane's colour within a vector
   ResHop<R> odd[P], even[P];
+  R dg[NR];
+#pragma unroll
+  for (int r = 0; r < NR; r++) dg[r] = (R)a.diag[r < a.nvec ? r : a.nvec - 1];
   C rv[P][NR], qv[P][NR];  // this lane's colour of r^(k-1) and r^(k-2)
 #pragma unroll
   for (int p = 0; p < P; p++) {
@@ -327,6 +330,7 @@ __device__ __forceinline__ void res_body(const ResArgs &a, int wg, int copy, lon
   if (threadIdx.x < NR) {
     const int r = threadIdx.x;
     const bool in = r < a.nvec;
+    s.diag[r] = in ? a.diag[r] : 0.0;
     s.rho1[r] = in ? a.sh[r].rho1 : 0.0;
     s.rho2[r] = 1.0;
     s.alpha[r] = 1.0;
@@ -434,7 +438,7 @@ __device__ __forceinline__ void res_body(const ResArgs &a, int wg, int copy, lon
       double h2 = 0.0;
       for (int q = 0; q < nw; q++) h2 += s.wave[1][q][r];
       const double rho1 = s.rho1[r], b = s.beta[r], ap = s.alpha[r];
-      const double mu2 = a.diag * rho1 + h2;
+      const double mu2 = s.diag[r] * rho1 + h2;
       const double pap = k >= 2 ? mu2 - b * rho1 / ap : mu2;
       const double alpha = rho1 / pap;
       s.coef[0][r] = alpha;
@@ -457,7 +461,7 @@ __device__ __forceinline__ void res_body(const ResArgs &a, int wg, int copy, lon
 #pragma unroll
         for (int q = 0; q < NB; q++) {
           const int r = r0 + q;
-          const R d = (R)a.diag, al = (R)s.coef[0][r], c1 = (R)s.coef[1][r];
+          const R d = dg[r], al = (R)s.coef[0][r], c1 = (R)s.coef[1][r];
           C x, rn;
           x.x = fmar(d, rv[p][r].x, (R)-0.5 * o[q].x);
           x.y = fmar(d, rv[p][r].y, (R)-0.5 * o[q].y);

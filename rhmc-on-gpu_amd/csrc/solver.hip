@@ -44,7 +44,7 @@ enum Slot {
   S_PARTIAL, S_SUMS, S_MS, S_CG, S_DIAG,
   S_R64, S_P64, S_S64, S_H64, S_PS64,
   S_B32, S_R32, S_P32, S_S32, S_H32, S_PS32, S_X32,
-  S_CR64, S_CX32, S_CR32, S_CP32, S_CS32, S_CH32,
+  S_CR64, S_CX32, S_CR32, S_CP32, S_CS32, S_CH32, S_CIDX,
   S_PW1, S_PW2, S_PW3, S_PWN,
   S_FH64,
   S_PARTIAL2, S_BASIS, S_BSH, S_HIST, S_COEF, S_HPART,
@@ -79,7 +79,7 @@ struct Workspace {
   GraphSlot group_graph[2];                    // the same for a group of lattices led by this context
   std::vector<DsArgs> group_tab;               // argument tables of the group's chunk (host copy)
   std::map<unsigned long long, int> group_tuned;  // lockstep launch shape per group composition
-  long basis_kmax[2] = {0, 0};                 // most basis iterations a FP32 / FP64 solve needed
+  long basis_kmax[3] = {0, 0, 0};              // most basis iterations a FP32 / FP64 solve, a correction needed
   int num_cu = 0;                              // compute units of the device
   bool resident_off = false;                   // a one-launch solve gave up waiting (device shared): not used again
   void *buf[S_COUNT] = {};
@@ -2001,15 +2001,15 @@ __global__ __launch_bounds__(kBlock) void k_cg_update_p(BlasArgs a) {
   }
 }
 
-// x64[j] += (double) x32[j]  (n elements of double2)
-__global__ __launch_bounds__(kBlock) void k_accum_f2d(double2 *x64, const float2 *x32, long n) {
+// vector idx[j] (idx null: j) of x64 += vector j = blockIdx.y of x32, n elements each
+__global__ __launch_bounds__(kBlock) void k_accum_f2d(double2 *x64, const float2 *x32, long n, const int *idx) {
   const long i = (long)blockIdx.x * kBlock + threadIdx.x;
+  const long j = blockIdx.y;
   if (i < n) {
-    const float2 v = x32[i];
-    double2 o = x64[i];
+    const float2 v = x32[j * n + i];
+    double2 &o = x64[(idx ? idx[j] : j) * n + i];
     o.x += (double)v.x;
     o.y += (double)v.y;
-    x64[i] = o;
   }
 }
 __global__ __launch_bounds__(kBlock) void k_copy_f2d(double2 *x64, const float2 *x32, long n) {
@@ -2066,6 +2066,7 @@ struct BmsArgs {
   long Vh;
   int nvec, nshift, cap;
   const double2 *b;
+  const int *bidx;      // right-hand side j is b's vector bidx[j] (null: j)
   void *basis;          // [cap][rhs][3][Vh]: slot k of every rhs contiguous
   double *partC;        // partials of rho_0
   int nbrC;
@@ -2091,9 +2092,10 @@ __global__ __launch_bounds__(kBlock) void k_bms_init(BmsArgs a) {
   site_range(Vh, bx, gridDim.x, h0, h1);
   double v[1] = {0.0};
   C *r0 = (C *)a.basis + (long)j * 3 * Vh;
+  const long jb = a.bidx ? a.bidx[j] : j;
   for (long h = h0 + threadIdx.x; h < h1; h += kBlock)
     for (int i = 0; i < 3; i++) {
-      const double2 bv = a.b[((long)j * 3 + i) * Vh + h];
+      const double2 bv = a.b[(jb * 3 + i) * Vh + h];
       const C cv = mk<R>((R)bv.x, (R)bv.y);
       r0[(long)i * Vh + h] = cv;
       v[0] += (double)cv.x * (double)cv.x + (double)cv.y * (double)cv.y;
@@ -2459,6 +2461,7 @@ struct FirstPass {
 // iterations (chunks of kChunk, replayed as HIP graphs) and the assembly.
 struct BasisRun {
   int nrhs = 0, nshift = 0, max_iter = 0;
+  int kind = 0;  // basis_kmax entry
   long cap = 0;
   void *basis = nullptr, *hh = nullptr;
   MsState *ms = nullptr;
@@ -2473,18 +2476,27 @@ struct BasisRun {
   bool resident = false;  // the iterations run as one launch
 };
 
+// Systems of a batch (the defect correction): right-hand side j is vector
+// idx[j] (device) of b and its operator MdagM + shift[j].
+struct SystemBatch {
+  const int *idx;
+  const double *shift;
+};
+
 // buffers, scalar state and the first launches; the iteration counter
 // iterc (device) is read by every launch of the iterations
 template <typename R, int LINK>
 static int bms_setup(Context &c, BasisRun &br, const double2 *b, int nrhs, int nshift, const double *shifts,
-                     const double *res_abs, int max_iter, int *iterc, double tol_abs = 0.0, double tol_rel = 0.0) {
+                     const double *res_abs, int max_iter, int *iterc, double tol_abs = 0.0, double tol_rel = 0.0,
+                     const SystemBatch *sys = nullptr) {
   using C = Cx<R>;
   const long Vh = c.Vh;
   const size_t vb = sizeof(C) * 3 * Vh;
   const bool dbl = sizeof(R) == 8;
   const size_t slot_bytes = vb * nrhs;
   const size_t have = c.ws->cap[S_BASIS];
-  long want = std::max<long>(kMinSlots, 2L * c.ws->basis_kmax[dbl ? 1 : 0]);
+  br.kind = sys ? 2 : dbl ? 1 : 0;
+  long want = std::max<long>(kMinSlots, 2L * c.ws->basis_kmax[br.kind]);
   long budget = (long)(have / slot_bytes);
   if (budget < want) {
     // growing: up to half of the free device memory (with the current basis),
@@ -2527,13 +2539,14 @@ static int bms_setup(Context &c, BasisRun &br, const double2 *b, int nrhs, int n
     for (int k = 0; k < nshift; k++) st.shift[k] = shifts[k];
   }
   std::vector<double> hd(nrhs, c.mass * c.mass);
+  for (int j = 0; sys && j < nrhs; j++) hd[j] += sys->shift[j];
   if (!h2d(c, br.ms, br.hs.data(), sizeof(MsState) * nrhs) || !h2d(c, br.diag, hd.data(), sizeof(double) * nrhs))
     return -1;
 
   BmsArgs &a = br.a;
   a = BmsArgs{};
   a.Vh = Vh; a.nvec = nrhs; a.nshift = nshift; a.cap = (int)cap;
-  a.b = b; a.basis = br.basis;
+  a.b = b; a.bidx = sys ? sys->idx : nullptr; a.basis = br.basis;
   a.partC = br.partC;
   a.sh = br.bsh; a.ms = br.ms;
   a.active = active_ptr(c);
@@ -2555,7 +2568,7 @@ static int bms_setup(Context &c, BasisRun &br, const double2 *b, int nrhs, int n
   hop.red = make_red(c, nrhs, EPI_STORE, nullptr, nullptr);
   hop.red.partial = br.partH;
   // live timing of the MD solver's hop (FP32, all pseudofermions)
-  br.timed = c.time_kernels && c.kt_clk && sizeof(R) == 4 && nrhs == c.n_pf && iterc == iter_ptr(c);
+  br.timed = c.time_kernels && c.kt_clk && sizeof(R) == 4 && nrhs == c.n_pf && iterc == iter_ptr(c) && !sys;
   DsArgs &mdm = br.mdm;
   mdm = hop;
   mdm.par_out = 0; mdm.in = br.hh; mdm.in_vs = 3 * Vh; mdm.out = nullptr; mdm.pin = br.basis; mdm.pin_vs = 3 * Vh;
@@ -2739,7 +2752,6 @@ template <typename R, int LINK>
 static int bms_finish(Context &c, BasisRun &br, double2 *x, int *iters_out, float2 *x32, bool asm_fp32,
                       BasisRestart *rs) {
   const long Vh = c.Vh;
-  const bool dbl = sizeof(R) == 8;
   const int nrhs = br.nrhs, nshift = br.nshift;
   const long cap = br.cap;
   // every coefficient index i < K <= iterations run < cap
@@ -2770,7 +2782,10 @@ static int bms_finish(Context &c, BasisRun &br, double2 *x, int *iters_out, floa
                        cst, (float *)nullptr, 0L, dklen);
     const dim3 grid((unsigned)((3 * Vh + kBlock - 1) / kBlock), nrhs);
     for (int s0 = 0; s0 < nshift; s0 += 16)
-      if (x32)
+      if (x32 && nshift <= 2)
+        hipLaunchKernelGGL((k_bms_assemble<R, 2, float2>), grid, dim3(kBlock), 0, c.stream, br.basis, dcoef, dklen,
+                           x32, Vh, (int)cst, nshift, s0, nrhs);
+      else if (x32)
         hipLaunchKernelGGL((k_bms_assemble<R, 16, float2>), grid, dim3(kBlock), 0, c.stream, br.basis, dcoef, dklen,
                            x32, Vh, (int)cst, nshift, s0, nrhs);
       else
@@ -2794,7 +2809,7 @@ static int bms_finish(Context &c, BasisRun &br, double2 *x, int *iters_out, floa
   }
   int kmax = 0;
   for (int j = 0; j < nrhs; j++) kmax = std::max(kmax, hs[j].iter);
-  long &kseen = c.ws->basis_kmax[dbl ? 1 : 0];
+  long &kseen = c.ws->basis_kmax[br.kind];
   kseen = std::max<long>(kseen, kmax);
   // the hop ran with work at iterations 1..kmax+1 (input slots 0..kmax);
   // slot kmax+1 holds the end of M^dag M(kmax+1) when a hop followed it
@@ -3023,7 +3038,7 @@ static int resident_launch(const std::vector<Context *> &cs, std::vector<BasisRu
       a.nvec = std::min(rl.nr, br.nrhs - r0); a.nshift = br.nshift; a.cap = (int)br.cap;
       a.part = part + (size_t)per * r0;
       a.abort = (int *)(part + np);
-      a.diag = c.mass * c.mass;
+      a.diag = br.diag + r0;
       a.sh = br.bsh + r0; a.ms = br.ms + r0; a.hist = br.hist + (size_t)r0 * br.cap * br.nshift;
       a.nwg = rl.nwg[q];
       a.sites = rl.sites[q];
@@ -3049,11 +3064,12 @@ static int resident_launch(const std::vector<Context *> &cs, std::vector<BasisRu
 template <typename R, int LINK>
 static int ms_cg_basis(Context &c, const double2 *b, int nrhs, int nshift, const double *shifts,
                        const double *res_abs, int max_iter, double2 *x, int *iters_out, float2 *x32,
-                       bool asm_fp32, BasisRestart *rs, double tol_abs = 0.0, double tol_rel = 0.0) {
+                       bool asm_fp32, BasisRestart *rs, double tol_abs = 0.0, double tol_rel = 0.0,
+                       const SystemBatch *sys = nullptr) {
   std::vector<BasisRun> runs(1);
   BasisRun &br = runs[0];
   int *iterc = iter_ptr(c);
-  int rc = bms_setup<R, LINK>(c, br, b, nrhs, nshift, shifts, res_abs, max_iter, iterc, tol_abs, tol_rel);
+  int rc = bms_setup<R, LINK>(c, br, b, nrhs, nshift, shifts, res_abs, max_iter, iterc, tol_abs, tol_rel, sys);
   if (rc) return rc;
   const std::vector<Context *> cs = {&c};
   if (const std::vector<ResidentLaunch> plan = resident_plan<R, LINK>(cs, runs); !plan.empty()) {
@@ -3066,7 +3082,7 @@ static int ms_cg_basis(Context &c, const double2 *b, int nrhs, int nshift, const
     if (rc != kResidentGaveUp) return rc;
     c.ws->resident_off = true;
     br = BasisRun();
-    rc = bms_setup<R, LINK>(c, br, b, nrhs, nshift, shifts, res_abs, max_iter, iterc, tol_abs, tol_rel);
+    rc = bms_setup<R, LINK>(c, br, b, nrhs, nshift, shifts, res_abs, max_iter, iterc, tol_abs, tol_rel, sys);
     if (rc) return rc;
   }
   GraphSlot &gs = c.ws->bms_graph[sizeof(R) == 8 ? 1 : 0];
@@ -3076,6 +3092,7 @@ static int ms_cg_basis(Context &c, const double2 *b, int nrhs, int nshift, const
   auto chunk = [&](bool eager) -> bool {
     memset(&key, 0, sizeof(key));
     key.a = br.a; key.hop = br.hop; key.mdm = br.mdm; key.nbr = br.nbr;
+    eager |= sys != nullptr;  // its right-hand sides differ from call to call; long launches
     key.a.b = nullptr;  // the right-hand sides are read only by k_bms_init, outside the chunk
     return chunk_run(c, gs, eager, &key, sizeof(key), [&]() { bms_chunk<R, LINK>(c, br, iterc, poll); });
   };
@@ -3351,7 +3368,8 @@ template <typename R, int LINK>
 static int ms_basis_solve(Context &c, const double2 *b, int nrhs, int nshift, const double *shifts,
                           const double *res_abs, int max_iter, double2 *x, int *iters_out, float2 *x32 = nullptr,
                           bool asm_fp32 = false, FirstPass *first = nullptr, double tol_abs = 0.0,
-                          double tol_rel = 0.0, std::vector<double> *bn2_out = nullptr) {
+                          double tol_rel = 0.0, std::vector<double> *bn2_out = nullptr,
+                          const SystemBatch *sys = nullptr) {
   using C = Cx<R>;
   BasisRestart rs;
   int it = 0;
@@ -3362,7 +3380,7 @@ static int ms_basis_solve(Context &c, const double2 *b, int nrhs, int nshift, co
     rs = first->rs;
   } else {
     rc = ms_cg_basis<R, LINK>(c, b, nrhs, nshift, shifts, res_abs, max_iter, x, &it, x32, asm_fp32, &rs, tol_abs,
-                              tol_rel);
+                              tol_rel, sys);
   }
   // the first pass's thresholds (continuations divide them by the largest |zeta|)
   std::vector<double> res_first;
@@ -3381,10 +3399,11 @@ static int ms_basis_solve(Context &c, const double2 *b, int nrhs, int nshift, co
     c.last_restarts++;
     const int n2 = (int)rs.rhs.size();
     std::vector<int> orig2(n2);
-    std::vector<double> scale2((size_t)n2 * nshift), res2(n2);
+    std::vector<double> scale2((size_t)n2 * nshift), res2(n2), shift2(n2);
     for (int q = 0; q < n2; q++) {
       const int j = rs.rhs[q];
       orig2[q] = orig[j];
+      if (sys) shift2[q] = sys->shift[orig2[q]];
       double zmax = 0.0;
       for (int s = 0; s < nshift; s++) {
         const double f = scale[(size_t)j * nshift + s] * rs.zeta[(size_t)q * nshift + s];
@@ -3407,8 +3426,10 @@ static int ms_basis_solve(Context &c, const double2 *b, int nrhs, int nshift, co
     if (!h2d(c, dorig, orig2.data(), sizeof(int) * n2) || !h2d(c, dscale, scale2.data(), sizeof(double) * scale2.size()))
       return -1;
     it = 0;
+    const SystemBatch sys2 = {nullptr, shift2.data()};
     rc = ms_cg_basis<R, LINK>(c, src, n2, nshift, shifts, res2.data(), std::max(1, max_iter - total),
-                              x32 ? nullptr : (double2 *)y, &it, x32 ? (float2 *)y : nullptr, asm_fp32, &rs);
+                              x32 ? nullptr : (double2 *)y, &it, x32 ? (float2 *)y : nullptr, asm_fp32, &rs, 0.0, 0.0,
+                              sys ? &sys2 : nullptr);
     total += it;
     if (rc < 0 || rc == kStatusNonFinite || rc == kBasisFull) return rc == kBasisFull ? -1 : rc;
     const dim3 grid((unsigned)((n3 + kBlock - 1) / kBlock), (unsigned)(n2 * nshift));
@@ -3428,7 +3449,8 @@ static int ms_basis_solve(Context &c, const double2 *b, int nrhs, int nshift, co
 }
 
 // batched CG on (MdagM + shift_j) e_j = r_j (FP32 iterations, FP32 links);
-// x32 receives e_j.
+// x32 receives e_j.  Where the stored basis is not used (explicit shifts, or
+// it does not fit): six launches per iteration, 15 passes over a vector.
 static int block_cg32(Context &c, const double2 *r64, int nsys, const double *shifts, const double *tol,
                       int max_iter, float2 *x32, int *iters_out) {
   const long Vh = c.Vh;
@@ -3494,6 +3516,64 @@ static int block_cg32(Context &c, const double2 *r64, int nsys, const double *sh
   return 0;
 }
 
+// One defect correction on the stored basis: x_j += e_j, (MdagM + shift_j)
+// e_j = r_j, for the systems with a tolerance below kTolMet (the others
+// have met their target), each a right-hand side with one shift of 0 and
+// its own operator.  An iteration is two launches and 6 passes over a vector
+// against the six launches and 15 passes of block_cg32, and a system's
+// solution is read off its residuals at the end: a solve of 24 systems of 24^3x8
+// takes 14.0 ms with block_cg32, 10.6 this way.  The systems go
+// in batches whose residuals fit kCorrectionBytes (or the basis there is),
+// at least 8 at a time so that a link is loaded once for as many.  A system
+// corrected before a batch finds no room (kBasisFull) has its tolerance set
+// to kTolMet.
+constexpr double kTolMet = 1e150;
+constexpr size_t kCorrectionBytes = 8ull << 30;
+static int correct_basis(Context &c, const double2 *r64, int nsys, const double *shifts, double *tol, int max_iter,
+                         double2 *x, float2 *e32, int *idx, int *iters_out) {
+  const long n = 3 * c.Vh;
+  std::vector<int> todo;
+  for (int j = 0; j < nsys; j++)
+    if (tol[j] < kTolMet) todo.push_back(j);
+  const size_t slots = (size_t)std::max<long>(kMinSlots, 2L * c.ws->basis_kmax[2]);
+  const size_t room = std::max(c.ws->cap[S_BASIS], kCorrectionBytes) / (slots * sizeof(float2) * (size_t)n);
+  const size_t most = std::max<size_t>(8, room);
+  const int restarts = c.last_restarts;  // counts the solve's own continuations
+  const std::string error = c.last_error;
+  const double zero = 0.0;
+  int rc = 0;
+  for (size_t q0 = 0; q0 < todo.size() && !rc; q0 += most) {
+    const int m = (int)std::min(most, todo.size() - q0);
+    std::vector<double> bs(m), bt(m);
+    for (int q = 0; q < m; q++) {
+      bs[q] = shifts[todo[q0 + q]];
+      bt[q] = tol[todo[q0 + q]];
+    }
+    if (!h2d(c, idx, &todo[q0], sizeof(int) * m)) return -1;
+    const SystemBatch sys = {idx, bs.data()};
+    int it = 0;
+    rc = ms_basis_solve<float, LINK_S12>(c, r64, m, 1, &zero, bt.data(), max_iter, nullptr, &it, e32, false, nullptr,
+                                         0.0, 0.0, nullptr, &sys);
+    if (rc == kStatusMaxCg) {  // the next cycle's true residuals decide
+      c.last_error = error;
+      rc = 0;
+    }
+    if (rc) break;
+    hipLaunchKernelGGL(k_accum_f2d, dim3((unsigned)((n + kBlock - 1) / kBlock), (unsigned)m), dim3(kBlock), 0,
+                       c.stream, x, e32, n, idx);
+    for (int q = 0; q < m; q++) tol[todo[q0 + q]] = kTolMet;
+    *iters_out = std::max(*iters_out, it);
+  }
+  c.last_restarts = restarts;
+  if (rc == kStatusNonFinite) c.last_error = "defect correction: non-finite value in the solver reductions";
+  return rc;
+}
+
+// the explicit-shift solver is selected
+static bool explicit_shifts(const Context &c) {
+  return c.ms_algorithm == 1 || getenv("RHMC_MS_EXPLICIT") != nullptr;
+}
+
 // r = b - ((m^2+shift_j) x_j - D_eo D_oe x_j) in FP64 with FP64 links; norms2[j]
 int residual_d(Context &c, const double2 *b, int b_group, const double2 *x, const double *shifts, int nvec,
                double2 *r, double *norms2) {
@@ -3536,7 +3616,9 @@ static int refine_fp64(Context &c, const double2 *b, int nrhs, int nshift, const
   double2 *r64 = (double2 *)ws_get(c, S_CR64, sizeof(double2) * 3 * Vh * nsys);
   if (!r64) return -1;
   float2 *e32 = nullptr;
+  int *idx = nullptr;
   int total_ref = 0;
+  bool basis = !explicit_shifts(c);
   double worst = 0.0;
   *ref_iters = 0;
   for (int cyc = 0;; cyc++) {
@@ -3553,18 +3635,28 @@ static int refine_fp64(Context &c, const double2 *b, int nrhs, int nshift, const
       worst = std::max(worst, rn / target);
       // inner FP32 solve: reduce this residual by ~1e-5, never below 0.5*target;
       // systems already converged get a huge tolerance (done at the first test)
-      tol[j] = rn <= target ? 1e150 : std::max(0.5 * target, 1e-5 * rn);
+      tol[j] = rn <= target ? kTolMet : std::max(0.5 * target, 1e-5 * rn);
       if (rn > target) ok = false;
     }
     c.last_true_res_max = worst;
     if (ok || cyc == 8) break;
     if (!e32 && !(e32 = (float2 *)ws_get(c, S_CX32, sizeof(float2) * 3 * Vh * nsys))) return -1;
-    int itc = 0;
-    const int rc = block_cg32(c, r64, nsys, sh.data(), tol.data(), max_iter, e32, &itc);
+    if (!idx && !(idx = (int *)ws_get(c, S_CIDX, sizeof(int) * kMaxRed))) return -1;
+    int itc = 0, rc = 0;
+    if (basis) {
+      rc = correct_basis(c, r64, nsys, sh.data(), tol.data(), max_iter, x, e32, idx, &itc);
+      if (rc == kBasisFull) basis = false;
+    }
+    if (!basis) {
+      int itb = 0;
+      rc = block_cg32(c, r64, nsys, sh.data(), tol.data(), max_iter, e32, &itb);
+      itc = std::max(itc, itb);
+      if (!rc)
+        hipLaunchKernelGGL(k_accum_f2d, dim3((unsigned)((3 * Vh + kBlock - 1) / kBlock), (unsigned)nsys), dim3(kBlock),
+                           0, c.stream, x, e32, 3 * Vh, (const int *)nullptr);
+    }
     if (rc) return rc;
     total_ref += itc;
-    hipLaunchKernelGGL(k_accum_f2d, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, c.stream, x,
-                       e32, n);
     c.last_refine_cycles = cyc + 1;
   }
   *ref_iters = total_ref;
@@ -3599,7 +3691,7 @@ static int ms_solve(Context &c, const double2 *b, int nrhs, int nshift, const do
   c.last_iters_refine = 0;
   c.last_restarts = 0;
   c.last_true_res_max = 0.0;
-  const bool explicit_shifts = c.ms_algorithm == 1 || getenv("RHMC_MS_EXPLICIT") != nullptr;
+  const bool by_shift = explicit_shifts(c);
   // |b| per rhs (relative residuals, the FP32 stage target, the FP64 checks).
   // The stored-basis pass forms it on the device and sets its own
   // thresholds there, max(tol_abs, tol_rel |b|), so the host waits for no
@@ -3619,10 +3711,10 @@ static int ms_solve(Context &c, const double2 *b, int nrhs, int nshift, const do
     set_norms(n2);
     return true;
   };
-  if ((explicit_shifts || first) && !host_norms()) return -1;
+  if ((by_shift || first) && !host_norms()) return -1;
   std::vector<double> dev_bn2;
   if (prec == PREC_FP64) {
-    int rc = explicit_shifts ? kBasisFull
+    int rc = by_shift ? kBasisFull
                              : ms_basis_solve<double, LINK_D12>(c, b, nrhs, nshift, shifts,
                                                                 have_norms ? res_abs.data() : nullptr, max_iter, x,
                                                                 iters, nullptr, false, first, rel ? 0.0 : res,
@@ -3657,7 +3749,7 @@ static int ms_solve(Context &c, const double2 *b, int nrhs, int nshift, const do
     for (int j = 0; j < nrhs; j++) res32[j] = std::max(res_abs[j], rel32 * sqrt(bn2[j]));
   int it32 = 0;
   const long n = 3 * Vh * (long)nrhs * nshift;
-  int rc = explicit_shifts ? kBasisFull
+  int rc = by_shift ? kBasisFull
                            : ms_basis_solve<float, LINK_S12>(c, b, nrhs, nshift, shifts,
                                                              have_norms ? res32.data() : nullptr, max_iter, x, &it32,
                                                              x32, prec == PREC_FP32, first, rel ? 0.0 : res,

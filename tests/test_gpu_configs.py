@@ -733,6 +733,45 @@ def test_one_launch_solves(dims, n_pf, monkeypatch):
             assert rel(x, y) < tol
 
 
+@pytest.mark.parametrize("dims,n_pf,n_shift", [((4, 4, 4, 4), 1, 1), ((8, 8, 8, 4), 3, 7), ((6, 10, 14, 6), 2, 5),
+                                               ((16, 16, 16, 16), 4, 24), ((24, 24, 24, 8), 1, 9)])
+def test_defect_correction_on_the_stored_basis(dims, n_pf, n_shift, monkeypatch):
+    """Mixed-precision solves, whose systems are corrected as right-hand sides
+    with an operator each: in one launch (few workgroups), in two launches per
+    iteration, with a last chunk that is not full, and in two batches (96
+    systems of 16^4).  Every true residual meets 1e-10 |b|; the solutions are
+    the FP64 solver's to 1e-9, as are those of the correction without a basis
+    (explicit shifts).  A second solve is the third bit for bit (the capacity
+    follows the first)."""
+    mass = 0.05
+    lat = fields.Lattice(*dims)
+    U = fields.random_links(lat, 41, 0.3)
+    phi = fields.gauss_spinor(lat, 42, n_pf)
+    b = np.geomspace(1e-4, 2.0, n_shift) if n_shift > 1 else np.array([1e-3])
+    bn = np.linalg.norm(phi.reshape(n_pf, -1), axis=1)
+    say("defect correction", dims, n_pf, n_shift)
+    g = Gpu(dims, mass=mass, n_pf=n_pf, max_order=n_shift)
+    g.init0(U)
+    g.init1(phi=phi)
+    g.multishift(b, 1e-11, relative=True, precision=0)
+    exact = g.get_fermions("smf")
+    for explicit in (True, False):
+        if explicit:
+            monkeypatch.setenv("RHMC_MS_EXPLICIT", "1")
+        else:
+            monkeypatch.delenv("RHMC_MS_EXPLICIT")
+        g.multishift(b, 1e-10, relative=True, precision=1)
+        assert (g.shifted_residuals(b) / bn[:, None]).max() <= 1e-10
+        x = g.get_fermions("smf")
+        for p, q in zip(x, exact):
+            assert rel(p, q) < 1e-9, explicit
+    g.multishift(b, 1e-10, relative=True, precision=1)
+    y = g.get_fermions("smf")
+    g.multishift(b, 1e-10, relative=True, precision=1)
+    assert np.array_equal(g.get_fermions("smf"), y)
+    g.close()
+
+
 @pytest.mark.parametrize("precision", [0, 2])
 def test_one_launch_solve_that_gives_up(precision, monkeypatch):
     """A one-launch solve whose waits are bounded at 0 ticks leaves (every
