@@ -258,6 +258,13 @@ template <typename T>
 __device__ __forceinline__ T ld_off(const T *base, unsigned byte_off) {
   return *(const T *)((const char *)base + byte_off);
 }
+// the same as a streaming (non-temporal) load: the line is the first to leave the caches
+template <typename T>
+__device__ __forceinline__ T ld_off_stream(const T *base, unsigned byte_off) {
+  using E = decltype(T::x);
+  typedef E V __attribute__((ext_vector_type(sizeof(T) / sizeof(E))));
+  return __builtin_bit_cast(T, __builtin_nontemporal_load((const V *)((const char *)base + byte_off)));
+}
 
 __device__ __forceinline__ Mat<double> load_link_d18(const double2 *__restrict__ U, long Vh, int mu, int par, long h) {
   Mat<double> m;

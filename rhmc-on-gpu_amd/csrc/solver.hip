@@ -716,14 +716,17 @@ struct LinkRaw {
   T e[N];
 };
 
-template <typename R, int LINK>
+// KEEP: directions whose links are loaded through the caches, the others' are
+// streamed (link_keep)
+template <typename R, int LINK, int KEEP>
 __device__ __forceinline__ void link_raw_load(const DsArgs &a, int mu, int par, int h, LinkRaw<R, LINK> &w) {
   using T = typename LinkRaw<R, LINK>::T;
   constexpr int N = LinkRaw<R, LINK>::N;
   const T *b = (const T *)a.U + (long)(mu * 2 + par) * N * a.L.Vh;
   const unsigned off = (unsigned)h * (unsigned)sizeof(T);
 #pragma unroll
-  for (int k = 0; k < N; k++) w.e[k] = ld_off(b + (long)k * a.L.Vh, off);
+  for (int k = 0; k < N; k++)
+    w.e[k] = mu < KEEP ? ld_off(b + (long)k * a.L.Vh, off) : ld_off_stream(b + (long)k * a.L.Vh, off);
 }
 
 template <typename R, int LINK>
@@ -759,13 +762,13 @@ struct HopIn {
 // hop k = 2 mu + (0 forward, 1 backward) of the site c (half index h):
 // forward  U_mu(x) psi(x+mu), link at x (output parity);
 // backward -U_mu(x-mu)^dag psi(x-mu), link at x-mu (the other parity)
-template <typename R, int LINK, int NR>
+template <typename R, int LINK, int NR, int KEEP = 4>
 __device__ __forceinline__ void hop_load(const DsArgs &a, const Cx<R> *const *inr, const SiteCoord &c, int h, int k,
                                          HopIn<R, LINK, NR> &d, bool spinors = true) {
   const int mu = k >> 1;
   const bool fwd = (k & 1) == 0;
   const int hn = neighbour_i(a.L, c, mu, fwd ? +1 : -1);
-  link_raw_load<R, LINK>(a, mu, fwd ? a.par_out : 1 - a.par_out, fwd ? h : hn, d.U);
+  link_raw_load<R, LINK, KEEP>(a, mu, fwd ? a.par_out : 1 - a.par_out, fwd ? h : hn, d.U);
   if (!spinors) return;
   const long Vh = a.L.Vh;
   const unsigned off = (unsigned)hn * (unsigned)sizeof(Cx<R>);
@@ -975,7 +978,7 @@ __device__ __forceinline__ void ds_site_out_bms(const DsArgs &a, const Cx<R> (&a
 
 // One workgroup (bid of nblk) of the one-lane Dslash: the body of k_dslash
 // and of the multi-lattice k_dslash_group.
-template <typename R, int LINK, int NR, int MODE, int RED>
+template <typename R, int LINK, int NR, int MODE, int RED, int KEEP = 4>
 __device__ __forceinline__ void ds_body(const DsArgs &a, unsigned bid, unsigned nblk) {
   using C = Cx<R>;
   if (MODE == DS_HOP && a.bms_ms)
@@ -1042,10 +1045,10 @@ __device__ __forceinline__ void ds_body(const DsArgs &a, unsigned bid, unsigned 
     C pv[MODE == DS_BMS ? NR : 1][3], qv[MODE == DS_BMS ? NR : 1][3];
     if constexpr (kBmsEarly) bms_site_loads<R, NR>(a, jbase, h, pinb, use_prev, pv, qv);
     HopIn<R, LINK, NR> buf[2];
-    hop_load<R, LINK, NR>(a, inr, c, h, 0, buf[0]);
+    hop_load<R, LINK, NR, KEEP>(a, inr, c, h, 0, buf[0]);
 #pragma unroll
     for (int k = 0; k < 8; k++) {
-      if (k + 1 < 8) hop_load<R, LINK, NR>(a, inr, c, h, k + 1, buf[(k + 1) & 1], k + 1 != 1 || !xrow);
+      if (k + 1 < 8) hop_load<R, LINK, NR, KEEP>(a, inr, c, h, k + 1, buf[(k + 1) & 1], k + 1 != 1 || !xrow);
       hop_apply<R, LINK, NR>(L, c, k, buf[k & 1], acc);
       if (k == 0 && xrow) xm_from_xp<R, LINK, NR>(buf[0], buf[1]);
       hop_fence<R, NR>(acc);
@@ -1063,6 +1066,35 @@ __device__ __forceinline__ void ds_body(const DsArgs &a, unsigned bid, unsigned 
 template <typename R, int LINK, int NR, int MODE, int RED>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(ds_waves<R, LINK, NR>()))) void k_dslash(DsArgs a) {
   ds_body<R, LINK, NR, MODE, RED>(a, blockIdx.x, gridDim.x);
+}
+
+// k_dslash with the links of directions >= KEEP streamed, for launches that
+// load every link once (all right-hand sides in one chunk)
+template <typename R, int LINK, int NR, int MODE, int RED, int KEEP>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(ds_waves<R, LINK, NR>()))) void k_dslash_stream(
+    DsArgs a) {
+  ds_body<R, LINK, NR, MODE, RED, KEEP>(a, blockIdx.x, gridDim.x);
+}
+
+// Directions whose links a launch keeps in the caches.  A solver iteration
+// reads every link twice; links larger than the 256 MiB Infinity Cache are
+// evicted before they come round again, and take the vectors with them.  So of
+// larger link fields only as many directions as fit half of that cache are
+// loaded through it, the others past it.  One iteration (hop and M^dag M, one
+// or two systems), us with all four directions kept and with the rule's:
+//   FP32 32^3x32  201 MB   89, 118 (all kept; 3: 91, 120, 1: 95, 134)
+//   FP32 48^3x12  255 MB  119 -> 114, 162 -> 148 (2 kept; 1: 120, 153)
+//   FP64 40^3x12  295 MB  148 -> 136, 196 -> 180 (1 kept; 2: 138, 185)
+//   FP64 48^3x12  510 MB  263 -> 227, 343 -> 309 (1 kept; none: 247, 307)
+//   FP32 64^3x16  805 MB  423 -> 384, 562 -> 512 (none; 1: 384, 532)
+//   FP64 64^3x16 1611 MB  837 -> 787, 1044 -> 1024 (none)
+// With several chunks a link is loaded again at once and streaming it costs
+// (8 systems of 32^3x8: 33 -> 37 us with 3 kept).
+constexpr size_t kInfinityCache = 256ull << 20;
+static int link_keep(size_t bytes) {
+  if (bytes <= kInfinityCache / 8 * 7) return 4;
+  const size_t keep = 4 * (kInfinityCache / 2) / bytes;
+  return keep >= 2 ? 2 : (int)keep;
 }
 
 // Dslash traversal order.  The hardware hands consecutive workgroups to the
@@ -1519,6 +1551,21 @@ static void dslash_prep(Context &c, DsArgs &a, int code) {
 }
 
 template <typename R, int LINK, int MODE, int RED>
+static void dslash_stream(Context &c, const DsArgs &a, dim3 grid, int nr, int keep) {
+#define DS_STREAM(NR, KEEP) \
+  hipLaunchKernelGGL((k_dslash_stream<R, LINK, NR, MODE, RED, KEEP>), grid, dim3(kBlock), 0, c.stream, a)
+  if (MODE != DS_POW && nr == 2) {
+    constexpr int NR = MODE == DS_POW ? 1 : 2;  // DS_POW: one vector
+    if (keep == 2) DS_STREAM(NR, 2);
+    else if (keep == 1) DS_STREAM(NR, 1);
+    else DS_STREAM(NR, 0);
+  } else if (keep == 2) DS_STREAM(1, 2);
+  else if (keep == 1) DS_STREAM(1, 1);
+  else DS_STREAM(1, 0);
+#undef DS_STREAM
+}
+
+template <typename R, int LINK, int MODE, int RED>
 static void dslash_launch(Context &c, DsArgs &a, int code) {
 #define DS_LAUNCH(KERNEL) hipLaunchKernelGGL(KERNEL, grid, dim3(kBlock), 0, c.stream, a)
   const int nr = shape_nr(code), lanes = shape_lanes(code) == 4 ? 4 : 1;
@@ -1526,6 +1573,8 @@ static void dslash_launch(Context &c, DsArgs &a, int code) {
   dim3 grid(a.nsb * a.nch);
   if constexpr (MODE == DS_POW) {  // one vector
     if (lanes == 4) DS_LAUNCH((k_dslash_ls<R, LINK, 1, MODE, RED>));
+    else if (const int keep = link_keep(sizeof(LinkRaw<R, LINK>) * 8 * (size_t)c.Vh); keep < 4)
+      dslash_stream<R, LINK, MODE, RED>(c, a, grid, 1, keep);
     else DS_LAUNCH((k_dslash<R, LINK, 1, MODE, RED>));
     return;
   }
@@ -1538,6 +1587,14 @@ static void dslash_launch(Context &c, DsArgs &a, int code) {
     }
     return;
   }
+  if constexpr (LINK != LINK_D18 && (MODE == DS_HOP || MODE == DS_BMS))
+    if (a.nch == 1 && nr <= 2) {
+      const int keep = link_keep(sizeof(LinkRaw<R, LINK>) * 8 * (size_t)c.Vh);
+      if (keep < 4) {
+        dslash_stream<R, LINK, MODE, RED>(c, a, grid, nr, keep);
+        return;
+      }
+    }
   switch (nr) {
     case 8: DS_LAUNCH((k_dslash<R, LINK, 8, MODE, RED>)); break;
     case 4: DS_LAUNCH((k_dslash<R, LINK, 4, MODE, RED>)); break;

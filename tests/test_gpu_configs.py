@@ -823,6 +823,40 @@ def test_power_iterations_in_one_launch(dims, monkeypatch):
     g.close()
 
 
+@pytest.mark.parametrize("dims,n_pf", [((40, 40, 40, 12), 2), ((48, 48, 48, 12), 1), ((64, 64, 64, 12), 2)])
+def test_streamed_links(dims, n_pf, monkeypatch):
+    """Lattices whose links exceed the Infinity Cache, where the launches of one
+    or two systems stream the links of some directions (FP64 of 40^3x12 and
+    48^3x12: three; FP32 of 48^3x12: two; 64^3x12: all).  Against the
+    lane-split kernels, which stream none: FP64 solutions to 4e-8 (both have
+    true residuals of 1e-10 |b|, eigenvalues in 0.09 .. 16.1), FP32 true
+    residuals to 1e-4 |b|, the largest eigenvalue to 1e-11."""
+    lat = fields.Lattice(*dims)
+    say("streamed links", dims, n_pf)
+    rng = np.random.default_rng(51)
+    U = fields.haar_su3(rng, 4096)[rng.integers(0, 4096, 4 * lat.V)]
+    U *= lat.eta()[:, None, None]
+    phi = fields.gauss_spinor(lat, 52, n_pf)
+    bn = np.linalg.norm(phi.reshape(n_pf, -1), axis=1)
+    b = np.array([1e-3, 1.0])
+    out = []
+    for shape in (f"{n_pf}x4", f"{n_pf}"):
+        monkeypatch.setenv("RHMC_DSLASH_NR", shape)
+        g = Gpu(dims, mass=0.3, n_pf=n_pf, max_order=2)
+        g.init0(U)
+        g.init1(phi=phi)
+        g.multishift(b, 1e-5, relative=True, precision=2)
+        assert (g.shifted_residuals(b) / bn[:, None]).max() <= 1e-4
+        g.multishift(b, 1e-10, relative=True, precision=0)
+        assert (g.shifted_residuals(b) / bn[:, None]).max() <= 1e-10
+        out.append((g.get_fermions("smf"), g.find_max(1e-3, seed=7)))
+        g.close()
+        say("done", shape)
+    for x, y in zip(out[0][0], out[1][0]):
+        assert rel(x, y) < 4e-8
+    assert abs(out[0][1] - out[1][1]) < 1e-11 * out[0][1]
+
+
 # ------------------------------------------------- large host transfers
 @pytest.mark.parametrize("dims", [(8, 8, 8, 4), (16, 14, 12, 6), (18, 16, 14, 10), (32, 32, 16, 8)])
 def test_host_transfers_round_trip(dims):
