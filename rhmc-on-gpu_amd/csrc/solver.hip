@@ -2193,8 +2193,8 @@ __global__ __launch_bounds__(kBlock) void k_bms_init_fin(BmsArgs a) {
   if (threadIdx.x == 0) a.active[0] = 0;
 }
 
-// x[j][s] (FP64) = sum_{i<K} coef[j][s][i] basis[j][i] for NS shifts per
-// pass; klen[j] = basis vectors of rhs j (slots beyond were never written).
+// x[j][s] (FP64) = sum_{i<K} coef[j][s][i] basis[j][i], NS shifts (group
+// blockIdx.z) per thread; klen[j] = basis vectors of rhs j (slots beyond were never written).
 // A tall-skinny product (3 Vh complex rows x K) . (K x NS real): one thread
 // per (colour, site) element streams its K basis values once, while the
 // workgroup stages the coefficients of kTileK basis indices in LDS, where
@@ -2205,14 +2205,14 @@ constexpr int kTileK = 32;
 
 template <typename R, int NS, typename XO>
 __global__ __launch_bounds__(kBlock) void k_bms_assemble(const void *basis, const double *coef, const int *klen,
-                                                         XO *x, long Vh, int cstride, int nshift, int s0, int nvec) {
+                                                         XO *x, long Vh, int cstride, int nshift, int nvec) {
   using C = Cx<R>;
   __shared__ double2 cs[kTileK][NS / 2];
   const long n3 = 3 * Vh;
   const long e = (long)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   const int j = blockIdx.y;
   const int kmax = klen[j];
-  const int ns = nshift - s0 < NS ? nshift - s0 : NS;
+  const int s0 = (int)blockIdx.z * NS, ns = nshift - s0 < NS ? nshift - s0 : NS;
   const long ss = (long)nvec * n3;  // slot stride
   const C *bj = (const C *)basis + (long)j * n3 + (e < n3 ? e : 0);
   const double *cj = coef + ((long)j * nshift + s0) * cstride;
@@ -2842,16 +2842,18 @@ static int bms_finish(Context &c, BasisRun &br, double2 *x, int *iters_out, floa
     hipLaunchKernelGGL(k_bms_coef, dim3(nshift, nrhs), dim3(64), 0, c.stream, br.ms, br.hist, cap, nshift, dcoef,
                        cst, (float *)nullptr, 0L, dklen);
     const dim3 grid((unsigned)((3 * Vh + kBlock - 1) / kBlock), nrhs);
-    for (int s0 = 0; s0 < nshift; s0 += 16)
-      if (x32 && nshift <= 2)
-        hipLaunchKernelGGL((k_bms_assemble<R, 2, float2>), grid, dim3(kBlock), 0, c.stream, br.basis, dcoef, dklen,
-                           x32, Vh, (int)cst, nshift, s0, nrhs);
-      else if (x32)
-        hipLaunchKernelGGL((k_bms_assemble<R, 16, float2>), grid, dim3(kBlock), 0, c.stream, br.basis, dcoef, dklen,
-                           x32, Vh, (int)cst, nshift, s0, nrhs);
-      else
-        hipLaunchKernelGGL((k_bms_assemble<R, 16, double2>), grid, dim3(kBlock), 0, c.stream, br.basis, dcoef, dklen,
-                           x, Vh, (int)cst, nshift, s0, nrhs);
+    // shifts per thread: 16 read the basis once; 4, over as many more
+    // workgroups, where those would leave CUs idle (8^3x4, 16 shifts: 24 -> 9
+    // us; 20x14x12x6 with two systems, 238 workgroups: 36 -> 28; 16^4, 384
+    // workgroups: 86 -> 125, not taken); 2 for FP32 solutions (the defect
+    // correction's, one shift each)
+#define ASSEMBLE(NS, XO, X)                                                                                    \
+  hipLaunchKernelGGL((k_bms_assemble<R, NS, XO>), dim3(grid.x, grid.y, (unsigned)((nshift + NS - 1) / NS)),    \
+                     dim3(kBlock), 0, c.stream, br.basis, dcoef, dklen, X, Vh, (int)cst, nshift, nrhs)
+    if (x32) ASSEMBLE(2, float2, x32);
+    else if ((int)(grid.x * grid.y) * ((nshift + 15) / 16) < c.ws->num_cu) ASSEMBLE(4, double2, x);
+    else ASSEMBLE(16, double2, x);
+#undef ASSEMBLE
   }
   if (!hip_ok(c, hipGetLastError(), "basis assemble")) return -1;
   // the systems' final state (after the assembly: one wait for both)

@@ -823,6 +823,30 @@ def test_power_iterations_in_one_launch(dims, monkeypatch):
     g.close()
 
 
+@pytest.mark.parametrize("dims,n_pf,n_shift", [((4, 4, 4, 4), 1, 1), ((6, 6, 4, 4), 3, 5), ((8, 8, 8, 4), 1, 17),
+                                               ((8, 8, 8, 4), 2, 32), ((12, 10, 8, 6), 9, 4)])
+def test_assembly_of_few_workgroups(dims, n_pf, n_shift):
+    """Shifted solutions of lattices whose assembly has fewer workgroups than
+    there are CUs (4 shifts per thread, a ragged last group), against the
+    oracle to 1e-9 (residuals of 1e-11 |b|, the smallest eigenvalue 0.01)."""
+    lat = fields.Lattice(*dims)
+    U = fields.random_links(lat, 61, 0.3)
+    phi = fields.gauss_spinor(lat, 62, n_pf)
+    b = np.geomspace(1e-3, 2.0, n_shift) if n_shift > 1 else np.array([1e-2])
+    say("assembly", dims, n_pf, n_shift)
+    g = Gpu(dims, mass=0.1, n_pf=n_pf, max_order=n_shift)
+    g.init0(U)
+    g.init1(phi=phi)
+    g.multishift(b, 1e-11, relative=True, precision=0)
+    x = g.get_fermions("smf").reshape(n_pf, n_shift, lat.Vh, 3)
+    g.close()
+    o = Oracle(dims)
+    for ps in range(n_pf):
+        xo, _ = o.multishift(U, 0.1, phi[ps], b, 1e-12 * np.linalg.norm(phi[ps]))
+        for k in range(n_shift):
+            assert rel(x[ps, k], xo[k]) < 1e-9, (ps, k)
+
+
 @pytest.mark.parametrize("dims,n_pf", [((40, 40, 40, 12), 2), ((48, 48, 48, 12), 1), ((64, 64, 64, 12), 2)])
 def test_streamed_links(dims, n_pf, monkeypatch):
     """Lattices whose links exceed the Infinity Cache, where the launches of one
