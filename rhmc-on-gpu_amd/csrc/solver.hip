@@ -2978,6 +2978,12 @@ static unsigned resident_wgs(const Context &c, int threads, int sites, int &nwg)
   return (unsigned)((nwg + 7) / 8 * 8);
 }
 
+// h of every iteration has a slot of its own, as r^(k) has in the basis
+template <typename R>
+static size_t resident_h_bytes(const Context &c, const BasisRun &br) {
+  return sizeof(Cx<R>) * (size_t)(3 * c.Vh * br.nrhs) * br.cap;
+}
+
 // The launches of a solve over one or several lattices; empty where the
 // launches per iteration are used.  Measured per iteration (us, one launch
 // against the two tuned launches; FP64, FP32):
@@ -3004,13 +3010,19 @@ static std::vector<ResidentLaunch> resident_plan(const std::vector<Context *> &c
   const unsigned cus = (unsigned)w.num_cu;
   int nvec = 0;
   bool split = true;  // every right-hand side's vectors are whole cache lines
+  size_t more = 0;    // device memory to be allocated for the h slots
   for (int l = 0; l < n; l++) {
+    const size_t need = resident_h_bytes<R>(*cs[l], runs[l]), have = cs[l]->ws->cap[S_RES_H];
+    if (need > have) more += need - have;
     const size_t vb = (size_t)3 * cs[l]->Vh * sizeof(Cx<R>);
     if (runs[l].timed || runs[l].nrhs * vb % 128) return {};
     if ((size_t)cs[l]->Vh * 8 * sizeof(LinkRaw<R, LINK>) >= (1ull << 32)) return {};
     nvec = std::max(nvec, runs[l].nrhs);
     split = split && vb % 128 == 0;
   }
+  // a device too full for a second set of slots keeps the launches per iteration
+  size_t fr = 0, tot = 0;
+  if (more && (hipMemGetInfo(&fr, &tot) != hipSuccess || more > fr / 2)) return {};
   auto all = [&](int nr, int threads, int sites) {
     ResidentLaunch r;
     r.nr = nr;
@@ -3084,7 +3096,7 @@ static int resident_launch(const std::vector<Context *> &cs, std::vector<BasisRu
     Context &c = *cs[rl.lat[q]];
     BasisRun &br = runs[rl.lat[q]];
     const long v = 3 * c.Vh;
-    Cx<R> *h = (Cx<R> *)ws_get(c, S_RES_H, sizeof(Cx<R>) * (size_t)(v * br.nrhs) * br.cap);
+    Cx<R> *h = (Cx<R> *)ws_get(c, S_RES_H, resident_h_bytes<R>(c, br));
     const int per = kResRing * kResCopies * res_copy(rl.nwg[q]), np = per * br.nrhs;
     unsigned long long *part = (unsigned long long *)ws_get(c, S_RES_PART, sizeof(unsigned long long) * np + 64);
     if (!h || !part) return -1;
@@ -3673,7 +3685,6 @@ static int refine_fp64(Context &c, const double2 *b, int nrhs, int nshift, const
                        const double *res_abs, int max_iter, double2 *x, int *ref_iters) {
   const long Vh = c.Vh;
   const int nsys = nrhs * nshift;
-  const long n = 3 * Vh * (long)nsys;
   std::vector<double> sh(nsys), nr2(nsys), tol(nsys);
   for (int j = 0; j < nsys; j++) sh[j] = shifts[j % nshift];
   double2 *r64 = (double2 *)ws_get(c, S_CR64, sizeof(double2) * 3 * Vh * nsys);
