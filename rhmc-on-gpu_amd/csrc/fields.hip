@@ -1144,15 +1144,19 @@ int time_copy(Context &c, size_t bytes, int reps, double *ms) {
 // takes 2.8 ms, and more threads or larger chunks gain nothing.
 //
 // The pinned buffers (16 MB) serve every context of the process, one
-// transfer at a time, and are freed with the last context.
+// transfer at a time, and are freed with the last context.  Allocating them
+// takes 3.5 ms, as long as they save on some 50 MB, so they are allocated by
+// the transfer that brings the large ones' total past kStageWorth.
 constexpr int kStageThreads = 4;
 constexpr size_t kStageChunk = 2u << 20;
 constexpr size_t kStageMin = 8u << 20;  // smaller copies: the runtime's (two chunks a thread and more)
+constexpr size_t kStageWorth = 64u << 20;
 
 struct HostStage {
   std::mutex m;
   char *buf = nullptr;
   int users = 0;
+  size_t moved = 0;  // bytes of the large transfers
 };
 static HostStage &host_stage() {
   static HostStage s;
@@ -1166,9 +1170,10 @@ void host_stage_retain() {
 void host_stage_release() {
   HostStage &s = host_stage();
   std::lock_guard<std::mutex> l(s.m);
-  if (--s.users == 0 && s.buf) {
-    hipHostFree(s.buf);
+  if (--s.users == 0) {
+    if (s.buf) hipHostFree(s.buf);
     s.buf = nullptr;
+    s.moved = 0;
   }
 }
 
@@ -1179,7 +1184,9 @@ static bool host_copy(Context &c, void *dev, void *host, size_t bytes, bool down
   std::unique_lock<std::mutex> l(s.m, std::defer_lock);
   if (bytes >= kStageMin) {
     l.lock();
-    if (!s.buf && hipHostMalloc((void **)&s.buf, 2 * kStageThreads * kStageChunk, hipHostMallocPortable) != hipSuccess) {
+    if (s.moved <= kStageWorth) s.moved += bytes;
+    if (!s.buf && s.moved > kStageWorth &&
+        hipHostMalloc((void **)&s.buf, 2 * kStageThreads * kStageChunk, hipHostMallocPortable) != hipSuccess) {
       (void)hipGetLastError();
       s.buf = nullptr;
     }
