@@ -21,6 +21,7 @@ SOURCES = [
 HEADERS = [
     os.path.join(HERE, "csrc", "lattice.hpp"),
     os.path.join(HERE, "csrc", "resident.hpp"),
+    os.path.join(HERE, "csrc", "resident_plan.hpp"),
     os.path.join(HERE, "csrc", "context.hpp"),
     os.path.join(ROOT, "include", "gpu.h"),
     os.path.join(ROOT, "include", "cu_inverter.h"),

@@ -34,6 +34,8 @@
 // with the per-iteration launches.
 #pragma once
 
+#include "resident_plan.hpp"
+
 namespace rhmc {
 
 constexpr int kResAborted = 2;            // MsState::nonfinite of system 0: the grid gave up
@@ -526,7 +528,6 @@ __device__ __forceinline__ void res_body(const ResArgs &a, int wg, int copy, lon
 // The grid is the concatenation of the members' grids, each a multiple of 8
 // so that each XCD (workgroups are dealt to the 8 XCDs in turn) has a
 // contiguous part of the sites; every member meets on its own.
-constexpr int kResMaxMembers = 22;
 struct ResGroup {
   ResArgs a[kResMaxMembers];
   unsigned start[kResMaxMembers + 1];

@@ -2953,15 +2953,6 @@ class ResidentShare {
   double s_;
 };
 
-// One launch of k_bms_resident: the lattices of a solve that share it
-// (indices), the right-hand sides per member, threads per workgroup, each
-// lattice's sites per lane and workgroups per member.
-struct ResidentLaunch {
-  int nr = 1, threads = 512, sites_max = 1;
-  std::vector<int> lat, sites, nwg;
-  unsigned total = 0;  // workgroups
-};
-
 template <typename R, int LINK, int NR, int P>
 static int resident_per_cu(int threads) {
   int n = 0;
@@ -2971,118 +2962,32 @@ static int resident_per_cu(int threads) {
   }
   return n;
 }
-// workgroups of a lattice's member, rounded up to the 8 XCDs
-static unsigned resident_wgs(const Context &c, int threads, int sites, int &nwg) {
-  const long per = (long)(threads / 4) * sites;
-  nwg = (int)((c.Vh + per - 1) / per);
-  return (unsigned)((nwg + 7) / 8 * 8);
-}
-
 // h of every iteration has a slot of its own, as r^(k) has in the basis
 template <typename R>
 static size_t resident_h_bytes(const Context &c, const BasisRun &br) {
   return sizeof(Cx<R>) * (size_t)(3 * c.Vh * br.nrhs) * br.cap;
 }
 
-// The launches of a solve over one or several lattices; empty where the
-// launches per iteration are used.  Measured per iteration (us, one launch
-// against the two tuned launches; FP64, FP32):
-//   8^3x4 1 to 8 systems  7.9 / 18,     7.5 / 18
-//   12^4  1               8.0 / 18,     7.0 / 17
-//   12^4  8 (4 a member) 19.9 / 28,    14.2 / 20
-//   16^4  1              12.0 / 22,     9.3 / 16
-//   16^4  2 (2 a member) 16.8 / 25,    12.5 / 18
-//   16^4  4 (4 a member) 25.4 / 28,    17.5 / 28
-//   16^4  8 (8 a member) 46   / 43,    32   / 28   (not taken)
-//   24^3x8 1 (two sites) 24.8 / 28,    17.7 / 19
-// The rule: the fewest systems per member (1, 2 or 4), then the smaller
-// workgroups, for which there is at most one workgroup per CU (16^4 with one
-// system: 14.5 us with 512 workgroups of 256 lanes).  One system on a lattice
-// too large for that may take two sites per lane (two systems of 16^4 that
-// way: 26 us).  Several lattices that do not fit that way
-// share the CUs as far as registers allow (the largest with two sites per
-// lane), else they run as up to three launches.
+// The launches of a solve over one or several lattices (resident_pack); empty
+// where the launches per iteration are used.
 template <typename R, int LINK>
 static std::vector<ResidentLaunch> resident_plan(const std::vector<Context *> &cs, const std::vector<BasisRun> &runs) {
   const Workspace &w = *cs[0]->ws;
-  const int n = (int)cs.size();
   if (w.resident_off || w.num_cu < 8 || getenv("RHMC_DSLASH_NR")) return {};
-  const unsigned cus = (unsigned)w.num_cu;
-  int nvec = 0;
-  bool split = true;  // every right-hand side's vectors are whole cache lines
-  size_t more = 0;    // device memory to be allocated for the h slots
-  for (int l = 0; l < n; l++) {
+  std::vector<ResidentLattice> ls;
+  size_t more = 0;  // device memory to be allocated for the h slots
+  for (size_t l = 0; l < cs.size(); l++) {
     const size_t need = resident_h_bytes<R>(*cs[l], runs[l]), have = cs[l]->ws->cap[S_RES_H];
     if (need > have) more += need - have;
     const size_t vb = (size_t)3 * cs[l]->Vh * sizeof(Cx<R>);
     if (runs[l].timed || runs[l].nrhs * vb % 128) return {};
     if ((size_t)cs[l]->Vh * 8 * sizeof(LinkRaw<R, LINK>) >= (1ull << 32)) return {};
-    nvec = std::max(nvec, runs[l].nrhs);
-    split = split && vb % 128 == 0;
+    ls.push_back({cs[l]->Vh, runs[l].nrhs, vb % 128 == 0});
   }
   // a device too full for a second set of slots keeps the launches per iteration
   size_t fr = 0, tot = 0;
   if (more && (hipMemGetInfo(&fr, &tot) != hipSuccess || more > fr / 2)) return {};
-  auto all = [&](int nr, int threads, int sites) {
-    ResidentLaunch r;
-    r.nr = nr;
-    r.threads = threads;
-    r.sites_max = sites;
-    r.sites.assign(n, sites);
-    r.nwg.resize(n);
-    int members = 0;
-    for (int l = 0; l < n; l++) {
-      const int m = (runs[l].nrhs + nr - 1) / nr;
-      members += m;
-      r.lat.push_back(l);
-      r.total += resident_wgs(*cs[l], threads, sites, r.nwg[l]) * m;
-    }
-    if (members > kResMaxMembers || (!split && nr < nvec)) r.total = ~0u;
-    return r;
-  };
-  for (int nr = 1; nr <= 4; nr *= 2)
-    for (int threads = 256; threads <= 512; threads *= 2)
-      if (const ResidentLaunch r = all(nr, threads, 1); r.total <= cus) return {r};
-  if (n == 1) {
-    if (nvec == 1)
-      if (const ResidentLaunch r = all(1, 512, 2); r.total <= cus) return {r};
-    return {};
-  }
-  // several lattices, one system per member: as many workgroups as the CUs
-  // hold, the largest lattices with two sites per lane until they fit
-  ResidentLaunch r = all(1, 512, 1);
-  if (r.total != ~0u) {
-    const unsigned room = cus * (unsigned)resident_per_cu<R, LINK, 1, 2>(512);
-    r.sites_max = 2;
-    while (r.total > room) {
-      int big = -1;
-      for (int l = 0; l < n; l++)
-        if (r.sites[l] == 1 && (big < 0 || cs[l]->Vh > cs[big]->Vh)) big = l;
-      if (big < 0) break;
-      r.total -= (unsigned)((r.nwg[big] + 7) / 8 * 8) * runs[big].nrhs;
-      r.sites[big] = 2;
-      r.total += resident_wgs(*cs[big], 512, 2, r.nwg[big]) * runs[big].nrhs;
-    }
-    if (r.total <= room) return {r};
-  }
-  // in turn: the largest first, each into the first launch with room for it
-  std::vector<int> order(n);
-  for (int l = 0; l < n; l++) order[l] = l;
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cs[a]->Vh > cs[b]->Vh; });
-  std::vector<ResidentLaunch> out;
-  for (const int l : order) {
-    int nwg = 0;
-    const unsigned t = resident_wgs(*cs[l], 512, 1, nwg) * (unsigned)runs[l].nrhs;
-    if (t > cus || !split) return {};
-    size_t q = 0;
-    while (q < out.size() && out[q].total + t > cus) q++;
-    if (q == out.size()) out.emplace_back();
-    out[q].lat.push_back(l);
-    out[q].sites.push_back(1);
-    out[q].nwg.push_back(nwg);
-    out[q].total += t;
-  }
-  return out.size() <= 3 ? out : std::vector<ResidentLaunch>();
+  return resident_pack(ls, (unsigned)w.num_cu, [] { return resident_per_cu<R, LINK, 1, 2>(512); });
 }
 
 // all iterations of the launch's lattices on the first context's stream
@@ -3104,6 +3009,10 @@ static int resident_launch(const std::vector<Context *> &cs, std::vector<BasisRu
                        np, (int *)(part + np));
     br.resident = true;
     for (int r0 = 0; r0 < br.nrhs; r0 += rl.nr) {
+      if (g.n == kResMaxMembers) {
+        c0.last_error = "one-launch solve: too many members";
+        return -1;
+      }
       ResArgs &a = g.a[g.n];
       a.L = c.L;
       a.U = link_ptr<LINK>(c);
@@ -4043,9 +3952,9 @@ static int power_resident(Context &c, const double2 *start, double tol, double p
   Workspace *w = c.ws;
   if (w->resident_off || w->num_cu < 8 || getenv("RHMC_DSLASH_NR")) return 1;
   int threads = 256, sites = 1, nwg = 0;
-  unsigned total = resident_wgs(c, threads, sites, nwg);
-  if (total > (unsigned)w->num_cu) total = resident_wgs(c, threads = 512, sites, nwg);
-  if (total > (unsigned)w->num_cu) total = resident_wgs(c, threads, sites = 2, nwg);
+  unsigned total = resident_wgs(c.Vh, threads, sites, nwg);
+  if (total > (unsigned)w->num_cu) total = resident_wgs(c.Vh, threads = 512, sites, nwg);
+  if (total > (unsigned)w->num_cu) total = resident_wgs(c.Vh, threads, sites = 2, nwg);
   if (total > (unsigned)w->num_cu) return 1;
   const long n = 3 * c.Vh;  // whole cache lines: V/2 is a multiple of 8
   double2 *p = (double2 *)ws_get(c, S_PW1, sizeof(double2) * n * (2 * kPowSmall + 1));

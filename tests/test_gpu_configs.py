@@ -363,6 +363,39 @@ def test_lockstep_first_on_fresh_handles():
         s.close()
 
 
+@pytest.mark.parametrize("lats", [[((8, 8, 8, 4), 8)] * 12, [((16, 16, 16, 16), 1)] + [((8, 8, 8, 4), 8)] * 3],
+                         ids=["twelve_of_8", "one_and_three_of_8"])
+def test_lockstep_of_more_systems_than_one_launch_lists(lats):
+    """Groups with more right-hand sides (96; 25) than the argument table of a
+    one-launch solve has members, which the CUs would have room for: each
+    lattice gets the trajectory it runs alone, Delta H to 1e-9 max(1, |Delta
+    H|) (one MD step: |Delta H| of 8 10^4), links to 1e-10 (FP64 solves)."""
+    kws, gpus, starts = [], [], []
+    for i, (d, n_pf) in enumerate(lats):
+        order = (16, 16, 16) if n_pf == 8 else (12, 8, 12)
+        first, md, last = rhmc_approximations(2, n_pf, *order)
+        g = Gpu(d, mass=0.05, beta=5.6, n_pf=n_pf, max_order=16)
+        starts.append(fields.random_links(fields.Lattice(*d), 170 + i, 0.3))
+        gpus.append(g)
+        kws.append(dict(n_flavours=2, no_md=1, integrator="omelyan", res_md=1e-10, res_metro=1e-10, relative=True,
+                        bounds=(0.02, 5.6), draw_fields=True, seed=90 + i, first=(first.a0, first.a, first.b),
+                        md=(md.a0, md.a, md.b), last=(last.a0, last.a, last.b)))
+    say("lockstep of many systems", len(lats), sum(n for _, n in lats))
+    alone = []
+    for g, U, kw in zip(gpus, starts, kws):
+        g.init0(U)
+        r = g.trajectory(**kw)
+        alone.append((r.delta_h, g.end(ipdot=False, momenta=False)[0]))
+        g.init0(U)
+    say("alone done")
+    res, st = multi_trajectory(gpus, kws)
+    assert st == [0] * len(lats)
+    for g, r, (dh, U) in zip(gpus, res, alone):
+        assert abs(r.delta_h - dh) < 1e-9 * max(1.0, abs(dh))
+        assert rel(g.end(ipdot=False, momenta=False)[0], U) < 1e-10
+        g.close()
+
+
 # ------------------------------------------------------------------ C5
 def test_c5_48c12_trajectory_delta_h():
     """C5: 48^3x12, Nf=2, am=0.01, beta=5.6, 2 pseudofermions, Omelyan 20
