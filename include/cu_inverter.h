@@ -52,6 +52,22 @@ int cu_last_solve_stats(rhmc_gpu_t h, int *iters_fp32, int *iters_refine, int *c
  * whose true residuals were checked (FP64 stored-basis and mixed solves). */
 int cu_solver_counters(rhmc_gpu_t h, int *restarts, int *graph_captures, double *true_res_max);
 
+/* The forms this handle's work took so far, no counterpart in the reference:
+ * counts[RHMC_COUNT_*], the first n of them.  A lockstep solve counts on the
+ * first handle of the group. */
+enum {
+  RHMC_COUNT_ONE_LAUNCH = 0, /* solver passes whose iterations ran as one launch (or up to three, by lattice) */
+  RHMC_COUNT_GAVE_UP,        /* one-launch solves and bounds that ran out of their wait and were repeated     */
+  RHMC_COUNT_POWER,          /* bounds whose power iterations ran many per launch                             */
+  RHMC_COUNT_STAGED,         /* host transfers through the pinned chunks                                      */
+  RHMC_COUNT_MEMBERS,        /* of the latest one-launch solver pass: members,                                */
+  RHMC_COUNT_MEMBER_RHS,     /*   right-hand sides per member,                                                */
+  RHMC_COUNT_LANES,          /*   lanes per workgroup,                                                        */
+  RHMC_COUNT_LANE_SITES,     /*   most sites per lane                                                         */
+  RHMC_COUNTS
+};
+int cu_path_counters(rhmc_gpu_t h, long long *counts, int n);
+
 #ifdef __cplusplus
 }
 #endif

@@ -740,6 +740,12 @@ int cu_solver_counters(rhmc_gpu_t h, int *restarts, int *graph_captures, double 
   return RHMC_OK;
 }
 
+int cu_path_counters(rhmc_gpu_t h, long long *counts, int n) {
+  if (!h || !counts || n < 1) return RHMC_EINVAL;
+  for (int i = 0; i < n && i < RHMC_COUNTS; i++) counts[i] = h->c.path[i];
+  return RHMC_OK;
+}
+
 int gpu_time_copy(rhmc_gpu_t h, double bytes, int reps, double *ms) {
   if (!h || !ms || bytes < 1024 || reps < 1) return RHMC_EINVAL;
   hipSetDevice(h->c.device);

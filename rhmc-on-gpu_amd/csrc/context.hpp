@@ -7,6 +7,7 @@
 #include <string>
 #include <vector>
 
+#include "cu_inverter.h"
 #include "lattice.hpp"
 
 namespace rhmc {
@@ -114,6 +115,7 @@ struct Context {
   std::vector<double> force_coef_held;
   const double *force_coef_dev = nullptr;
   int graph_captures = 0;          // solver chunk graphs captured (instantiated) so far
+  long long path[RHMC_COUNTS] = {};  // cu_path_counters
 };
 
 // ------------------------------------------------------------------ launches

@@ -1196,6 +1196,7 @@ static bool host_copy(Context &c, void *dev, void *host, size_t bytes, bool down
                               : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, c.stream);
     return hip_ok(c, e, "host transfer");
   }
+  c.path[RHMC_COUNT_STAGED]++;
   const size_t n = (bytes + kStageChunk - 1) / kStageChunk;
   std::atomic<size_t> next{0};
   std::atomic<bool> ok{true};

@@ -28,7 +28,8 @@
 //   no L1 or L2 can hold an older copy of a line;
 // * partials and the abort flag are read with agent-scope atomic loads.
 //
-// A wait is bounded (ResGroup::wait): when it runs out (the grid is not
+// A wait is bounded (ResGroup::wait; 0: up at the first empty slot): when it
+// runs out (the grid is not
 // resident because another process holds the device) the workgroup sets the
 // abort flag and leaves, the others follow, and the host repeats the solve
 // with the per-iteration launches.
@@ -162,8 +163,8 @@ __device__ __forceinline__ bool res_wait(const ResArgs &a, ResShared<NR> &s, int
       for (int r = 0; r < NR; r++) none |= b[r] == kResNone;
       if (!none) break;
       if (n == 0) t0 = wall_clock64();
-      if ((n & 63) == 63 &&
-          (wall_clock64() - t0 > wait ||
+      if (((n & 63) == 63 || wait == 0) &&
+          (wall_clock64() - t0 >= wait ||
            __hip_atomic_load(a.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
         __hip_atomic_store(a.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         s.aborted = 1;

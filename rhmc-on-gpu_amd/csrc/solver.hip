@@ -2990,6 +2990,17 @@ static std::vector<ResidentLaunch> resident_plan(const std::vector<Context *> &c
   return resident_pack(ls, (unsigned)w.num_cu, [] { return resident_per_cu<R, LINK, 1, 2>(512); });
 }
 
+static void resident_count(Context &c, const std::vector<ResidentLaunch> &plan) {
+  c.path[RHMC_COUNT_ONE_LAUNCH]++;
+  c.path[RHMC_COUNT_MEMBERS] = c.path[RHMC_COUNT_LANE_SITES] = 0;
+  for (const ResidentLaunch &rl : plan) {
+    c.path[RHMC_COUNT_MEMBERS] += rl.members;
+    c.path[RHMC_COUNT_MEMBER_RHS] = rl.nr;
+    c.path[RHMC_COUNT_LANES] = rl.threads;
+    for (const int s : rl.sites) c.path[RHMC_COUNT_LANE_SITES] = std::max<long long>(c.path[RHMC_COUNT_LANE_SITES], s);
+  }
+}
+
 // all iterations of the launch's lattices on the first context's stream
 template <typename R, int LINK>
 static int resident_launch(const std::vector<Context *> &cs, std::vector<BasisRun> &runs, const ResidentLaunch &rl) {
@@ -3059,11 +3070,13 @@ static int ms_cg_basis(Context &c, const double2 *b, int nrhs, int nshift, const
   if (const std::vector<ResidentLaunch> plan = resident_plan<R, LINK>(cs, runs); !plan.empty()) {
     {
       ResidentShare share(c.device, (double)plan[0].total / c.ws->num_cu);
+      resident_count(c, plan);
       rc = resident_launch<R, LINK>(cs, runs, plan[0]);
       if (!rc) rc = bms_finish<R, LINK>(c, br, x, iters_out, x32, asm_fp32, rs);
       if (rc < 0) hipStreamSynchronize(c.stream);  // nothing of it in flight when the share is given back
     }
     if (rc != kResidentGaveUp) return rc;
+    c.path[RHMC_COUNT_GAVE_UP]++;
     c.ws->resident_off = true;
     br = BasisRun();
     rc = bms_setup<R, LINK>(c, br, b, nrhs, nshift, shifts, res_abs, max_iter, iterc, tol_abs, tol_rel, sys);
@@ -3261,11 +3274,13 @@ static int ms_cg_basis_group(std::vector<Context *> &cs, std::vector<GroupJob> &
       unsigned most = 0;
       for (const ResidentLaunch &rl : plan) most = std::max(most, rl.total);
       ResidentShare share(c0.device, std::min(1.0, (double)most / c0.ws->num_cu));
+      resident_count(c0, plan);
       for (size_t q = 0; q < plan.size() && !rc; q++) rc = resident_launch<R, LINK>(cs, runs, plan[q]);
       if (!rc) rc = finish();
       if (rc) hipStreamSynchronize(c0.stream);
     }
     if (rc != kResidentGaveUp) return rc;
+    c0.path[RHMC_COUNT_GAVE_UP]++;
     c0.ws->resident_off = true;
     if ((rc = setup())) return rc;
   }
@@ -3978,6 +3993,7 @@ static int power_resident(Context &c, const double2 *start, double tol, double p
   a.norms = pn; a.n = kPowSmall;
   const char *wait = getenv("RHMC_RESIDENT_WAIT");
   a.wait = wait ? atoll(wait) : kResWaitTicks;
+  c.path[RHMC_COUNT_POWER]++;
   ResidentShare share(c.device, (double)total / w->num_cu);
   double h[kPowSmall + 2];
   for (int i0 = 1;; i0 += kPowSmall) {
@@ -3988,6 +4004,7 @@ static int power_resident(Context &c, const double2 *start, double tol, double p
     if (!d2h_sync(c, h, pn, sizeof(double) * (kPowSmall + 2))) return -1;
     const int ran = (int)h[kPowSmall + 1];
     if (ran < 0) {
+      c.path[RHMC_COUNT_GAVE_UP]++;
       w->resident_off = true;
       return 1;
     }

@@ -137,6 +137,7 @@ def _declare(L):
         "cu_shifted_residuals": (I, [VP, I, VP, VP]),
         "cu_last_solve_stats": (I, [VP, PI, PI, PI]),
         "cu_solver_counters": (I, [VP, PI, PI, PD]),
+        "cu_path_counters": (I, [VP, VP, I]),
     }
     for name, (res, args) in sig.items():
         f = getattr(L, name)
@@ -385,6 +386,18 @@ class Gpu:
         a, b, c = C.c_int(), C.c_int(), C.c_double()
         self.L.cu_solver_counters(self.h, C.byref(a), C.byref(b), C.byref(c))
         return a.value, b.value, c.value
+
+    PATHS = ("one_launch", "gave_up", "power", "staged", "members", "member_rhs", "lanes", "lane_sites")
+
+    def path_counters(self):
+        """The forms this handle's work took so far (cu_path_counters): solver
+        passes run as one launch, those and bounds that gave up waiting, bounds
+        of many power iterations per launch, host transfers through the pinned
+        chunks; and the latest one-launch pass's members, right-hand sides per
+        member, lanes per workgroup and most sites per lane."""
+        v = (C.c_longlong * len(self.PATHS))()
+        self._check(self.L.cu_path_counters(self.h, v, len(self.PATHS)), "cu_path_counters")
+        return dict(zip(self.PATHS, v))
 
     def fermion_force(self, numerators, accumulate=False):
         num = np.ascontiguousarray(numerators, np.float64)

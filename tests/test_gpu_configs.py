@@ -832,6 +832,98 @@ def test_one_launch_solve_that_gives_up(precision, monkeypatch):
     assert rel(xs[0], xs[1]) < (1e-9 if precision == 0 else 2e-4)
 
 
+# members, right-hand sides per member, lanes and sites per lane in FP64 and FP32 (None: launches per iteration)
+@pytest.mark.parametrize("dims,n_pf,forms", [
+    ((4, 4, 4, 4), 1, [(1, 1, 256, 1)] * 2), ((6, 4, 4, 6), 3, [(3, 1, 256, 1)] * 2),
+    ((6, 6, 6, 6), 1, [(1, 1, 256, 1), None]), ((6, 6, 6, 6), 2, [(2, 1, 256, 1), (1, 2, 256, 1)]),
+    ((8, 8, 8, 4), 8, [(8, 1, 256, 1)] * 2), ((20, 14, 12, 6), 2, [(2, 1, 512, 1)] * 2),
+    ((20, 14, 12, 6), 4, [(2, 2, 512, 1)] * 2), ((16, 16, 16, 16), 1, [(1, 1, 512, 1)] * 2),
+    ((16, 16, 16, 16), 2, [(1, 2, 512, 1)] * 2), ((16, 16, 16, 16), 3, [(1, 4, 512, 1)] * 2),
+    ((16, 16, 16, 16), 8, [None] * 2), ((18, 16, 16, 16), 1, [(1, 1, 512, 2)] * 2),
+    ((24, 24, 24, 8), 1, [(1, 1, 512, 2)] * 2), ((24, 24, 24, 12), 1, [None] * 2)])
+def test_one_launch_solves_take_their_form(dims, n_pf, forms, monkeypatch):
+    """Which solves run their iterations as one launch on a device of 256
+    compute units, and over how many members; none do with a forced launch
+    shape.  (Whether their solutions are right: test_one_launch_solves.)"""
+    lat = fields.Lattice(*dims)
+    U = fields.random_links(lat, 35, 0.3)
+    phi = fields.gauss_spinor(lat, 36, n_pf)
+    say("form", dims, n_pf)
+    for forced in (False, True):
+        if forced:
+            monkeypatch.setenv("RHMC_DSLASH_NR", "1")
+        g = Gpu(dims, mass=0.1, n_pf=n_pf, max_order=2)
+        g.init0(U)
+        g.init1(phi=phi)
+        for prec, form in zip((0, 2), forms):
+            before = g.path_counters()["one_launch"]
+            g.multishift([1e-2, 1.0], 1e-5, relative=True, precision=prec)
+            c = g.path_counters()
+            assert (c["one_launch"] > before) == (form is not None and not forced)
+            if form and not forced:
+                assert (c["members"], c["member_rhs"], c["lanes"], c["lane_sites"]) == form
+        assert c["gave_up"] == 0
+        g.close()
+
+
+@pytest.mark.parametrize("precision", [0, 2])
+def test_one_launch_work_that_does_not_wait_is_repeated(precision, monkeypatch):
+    """A bound of 0 ticks: some workgroup finds an empty slot and gives up, the
+    others follow and every one exits.  The solve, a lockstep solve of two
+    lattices and the bounds are then repeated with the launches per iteration,
+    each counted, with the results of an unbounded run (solutions 1e-9 in FP64,
+    2e-4 in FP32; trajectories' links 1e-9; bounds 1e-11 of the largest)."""
+    dims, mass = (16, 16, 16, 16), 0.1
+    lat = fields.Lattice(*dims)
+    U = fields.random_links(lat, 37, 0.3)
+    phi = fields.gauss_spinor(lat, 38, 1)
+    b = np.geomspace(1e-3, 2.0, 5)
+    first, md, last = rhmc_approximations(2, 1, 6, 5, 6)
+    kw = dict(n_flavours=2, no_md=1, integrator="omelyan", res_md=1e-10, res_metro=1e-10, relative=True,
+              bounds=(0.02, 5.6), draw_fields=True, first=(first.a0, first.a, first.b), md=(md.a0, md.a, md.b),
+              last=(last.a0, last.a, last.b))
+    out = []
+    for wait in ("0", None):
+        if wait is None:
+            monkeypatch.delenv("RHMC_RESIDENT_WAIT")
+        else:
+            monkeypatch.setenv("RHMC_RESIDENT_WAIT", wait)
+        say("wait", wait, precision)
+        g = Gpu(dims, mass=mass, max_order=6)
+        g.init0(U)
+        g.init1(phi=phi)
+        g.multishift(b, 1e-10 if precision == 0 else 1e-6, relative=True, precision=precision)
+        x = g.get_fermions("smf")
+        c = g.path_counters()
+        assert c["one_launch"] >= 1 and c["gave_up"] == (0 if wait is None else 1)
+        g.close()
+        say("solve done")
+        g = Gpu(dims, mass=mass, max_order=6)
+        g.init0(U)
+        mx = g.find_max(1e-4, seed=3)
+        c = g.path_counters()
+        assert c["power"] == 1 and c["gave_up"] == (0 if wait is None else 1)
+        say("bounds done")
+        g.close()
+        gs = [Gpu(d, mass=mass, max_order=6) for d in (dims, (8, 8, 8, 4))]
+        links = []
+        for i, h in enumerate(gs):
+            h.init0(fields.random_links(fields.Lattice(*h.dims), 39 + i, 0.3))
+        res, st = multi_trajectory(gs, [dict(seed=5 + i, **kw) for i in range(2)])
+        assert st == [0, 0]
+        c = gs[0].path_counters()
+        assert c["one_launch"] >= 1 and c["gave_up"] == (0 if wait is None else 1)
+        for h in gs:
+            links.append(h.end(ipdot=False, momenta=False)[0])
+            h.close()
+        say("lockstep done")
+        out.append((x, mx, links))
+    (x0, m0, l0), (x1, m1, l1) = out
+    assert rel(x0, x1) < (1e-9 if precision == 0 else 2e-4)
+    assert abs(m0 - m1) < 1e-11 * m1
+    assert all(rel(p, q) < 1e-9 for p, q in zip(l0, l1))
+
+
 @pytest.mark.parametrize("dims", [(4, 4, 4, 4), (6, 4, 4, 6), (6, 6, 6, 6), (20, 14, 12, 6), (16, 16, 16, 16),
                                   (18, 16, 16, 16), (24, 24, 24, 12)])
 def test_power_iterations_in_one_launch(dims, monkeypatch):
