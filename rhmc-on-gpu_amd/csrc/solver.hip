@@ -160,6 +160,33 @@ static void *ws_get(Context &c, int slot, size_t bytes) {
   return p;
 }
 
+// free device memory as the sizing rules see it (RHMC_FREE_BYTES: at most that much)
+static size_t device_free() {
+  size_t fr = 0, tot = 0;
+  if (hipMemGetInfo(&fr, &tot) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  if (const char *e = getenv("RHMC_FREE_BYTES")) fr = std::min(fr, (size_t)strtoull(e, nullptr, 10));
+  return fr;
+}
+
+// A buffer that a faster form of some work needs beyond what its plain form
+// does: null, with no error left, where its growth would take more than half
+// of the free device memory or cannot be allocated.
+static void *ws_try(Context &c, int slot, size_t bytes) {
+  Workspace *w = c.ws;
+  if (w->cap[slot] >= bytes) return w->buf[slot];
+  if (bytes - w->cap[slot] > device_free() / 2) return nullptr;
+  const std::string error = c.last_error;
+  void *p = ws_get(c, slot, bytes);
+  if (!p) {
+    (void)hipGetLastError();
+    c.last_error = error;
+  }
+  return p;
+}
+
 // host -> device through the pinned ring, enqueued on c.stream
 bool h2d(Context &c, void *dst, const void *src, size_t bytes) {
   Workspace *w = c.ws;
@@ -3972,11 +3999,13 @@ static int power_resident(Context &c, const double2 *start, double tol, double p
   if (total > (unsigned)w->num_cu) total = resident_wgs(c.Vh, threads, sites = 2, nwg);
   if (total > (unsigned)w->num_cu) return 1;
   const long n = 3 * c.Vh;  // whole cache lines: V/2 is a multiple of 8
-  double2 *p = (double2 *)ws_get(c, S_PW1, sizeof(double2) * n * (2 * kPowSmall + 1));
+  // 129 vectors, at most 400 MB, where the launches take three
+  double2 *p = (double2 *)ws_try(c, S_PW1, sizeof(double2) * n * (2 * kPowSmall + 1));
+  if (!p) return 1;
   double *pn = (double *)ws_get(c, S_PWN, sizeof(double) * (kPowSmall + 2));
   const int np = kResRing * kResCopies * res_copy(nwg);
   unsigned long long *part = (unsigned long long *)ws_get(c, S_RES_PART, sizeof(unsigned long long) * np + 64);
-  if (!p || !pn || !part) return -1;
+  if (!pn || !part) return -1;
   hipMemcpyAsync(p, start, sizeof(double2) * n, hipMemcpyDeviceToDevice, c.stream);
   norm2_to(c, p, n, pn);
   PowArgs a = {};
@@ -4001,7 +4030,8 @@ static int power_resident(Context &c, const double2 *start, double tol, double p
                        np, a.r.abort);
     if (sites == 1) hipLaunchKernelGGL(k_pow_resident<1>, dim3(total), dim3(threads), 0, c.stream, a);
     else hipLaunchKernelGGL(k_pow_resident<2>, dim3(total), dim3(threads), 0, c.stream, a);
-    if (!d2h_sync(c, h, pn, sizeof(double) * (kPowSmall + 2))) return -1;
+    if (!hip_ok(c, hipGetLastError(), "power iterations") || !d2h_sync(c, h, pn, sizeof(double) * (kPowSmall + 2)))
+      return -1;
     const int ran = (int)h[kPowSmall + 1];
     if (ran < 0) {
       c.path[RHMC_COUNT_GAVE_UP]++;

@@ -948,6 +948,28 @@ def test_power_iterations_in_one_launch(dims, monkeypatch):
     g.close()
 
 
+@pytest.mark.parametrize("dims", [(4, 4, 4, 4), (16, 16, 16, 16), (24, 24, 24, 8)])
+def test_power_iterations_without_room_for_their_slots(dims, monkeypatch):
+    """Where the 129 vectors of the many-per-launch form would take more than
+    half of the free device memory, the bounds run two launches per iteration
+    on three vectors: the same bounds to 1e-11 of the largest, no error."""
+    lat = fields.Lattice(*dims)
+    U = fields.random_links(lat, 42, 0.3)
+    vectors = 129 * 48 * lat.Vh
+    say("power iterations, room", dims)
+    got = []
+    for room, taken in ((vectors, 0), (2 * vectors, 2)):
+        monkeypatch.setenv("RHMC_FREE_BYTES", str(room))
+        g = Gpu(dims, mass=0.05)
+        g.init0(U)
+        mx = g.find_max(1e-4, seed=5)
+        got.append((mx, g.find_min(mx, 1e-4, seed=6)))
+        assert g.path_counters()["power"] == taken
+        g.close()
+    for a, b in zip(*got):
+        assert abs(a - b) < 1e-11 * got[0][0]
+
+
 @pytest.mark.parametrize("dims,n_pf,n_shift", [((4, 4, 4, 4), 1, 1), ((6, 6, 4, 4), 3, 5), ((8, 8, 8, 4), 1, 17),
                                                ((8, 8, 8, 4), 2, 32), ((12, 10, 8, 6), 9, 4)])
 def test_assembly_of_few_workgroups(dims, n_pf, n_shift):
