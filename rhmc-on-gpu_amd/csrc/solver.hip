@@ -2551,6 +2551,7 @@ struct BasisRun {
   int nrhs = 0, nshift = 0, max_iter = 0;
   int kind = 0;  // basis_kmax entry
   long cap = 0;
+  long expect = 0;  // slots the iterations seen so far ask for
   void *basis = nullptr, *hh = nullptr;
   MsState *ms = nullptr;
   BmsShared *bsh = nullptr;
@@ -2585,14 +2586,12 @@ static int bms_setup(Context &c, BasisRun &br, const double2 *b, int nrhs, int n
   const size_t have = c.ws->cap[S_BASIS];
   br.kind = sys ? 2 : dbl ? 1 : 0;
   long want = std::max<long>(kMinSlots, 2L * c.ws->basis_kmax[br.kind]);
+  br.expect = want;
   long budget = (long)(have / slot_bytes);
-  if (budget < want) {
+  if (budget < want)
     // growing: up to half of the free device memory (with the current basis),
     // at most kMaxBasisBytes
-    size_t fr = 0, tot = 0;
-    hipMemGetInfo(&fr, &tot);
-    budget = (long)(std::min((fr + have) / 2, std::max(have, kMaxBasisBytes)) / slot_bytes);
-  }
+    budget = (long)(std::min((device_free() + have) / 2, std::max(have, kMaxBasisBytes)) / slot_bytes);
   want = std::max<long>(want, (long)(have / slot_bytes));
   long cap = std::min<long>(std::min<long>((long)max_iter + 2, kMaxSlots), std::min<long>(budget, want));
   if (const char *e = getenv("RHMC_BASIS_CAP")) cap = std::min<long>(cap, std::max(atol(e), kMinBasis));
@@ -2989,32 +2988,38 @@ static int resident_per_cu(int threads) {
   }
   return n;
 }
-// h of every iteration has a slot of its own, as r^(k) has in the basis
-template <typename R>
-static size_t resident_h_bytes(const Context &c, const BasisRun &br) {
-  return sizeof(Cx<R>) * (size_t)(3 * c.Vh * br.nrhs) * br.cap;
-}
-
 // The launches of a solve over one or several lattices (resident_pack); empty
-// where the launches per iteration are used.
+// where the launches per iteration are used.  A run that is placed has its
+// slots bounded by those its iterations so far ask for (the basis allocation
+// may hold many more, of a solve with more systems: h would be as large again)
+// and the h slots allocated; one that fills them is continued.
 template <typename R, int LINK>
-static std::vector<ResidentLaunch> resident_plan(const std::vector<Context *> &cs, const std::vector<BasisRun> &runs) {
+static std::vector<ResidentLaunch> resident_plan(const std::vector<Context *> &cs, std::vector<BasisRun> &runs) {
   const Workspace &w = *cs[0]->ws;
   if (w.resident_off || w.num_cu < 8 || getenv("RHMC_DSLASH_NR")) return {};
   std::vector<ResidentLattice> ls;
-  size_t more = 0;  // device memory to be allocated for the h slots
   for (size_t l = 0; l < cs.size(); l++) {
-    const size_t need = resident_h_bytes<R>(*cs[l], runs[l]), have = cs[l]->ws->cap[S_RES_H];
-    if (need > have) more += need - have;
     const size_t vb = (size_t)3 * cs[l]->Vh * sizeof(Cx<R>);
     if (runs[l].timed || runs[l].nrhs * vb % 128) return {};
     if ((size_t)cs[l]->Vh * 8 * sizeof(LinkRaw<R, LINK>) >= (1ull << 32)) return {};
     ls.push_back({cs[l]->Vh, runs[l].nrhs, vb % 128 == 0});
   }
+  std::vector<ResidentLaunch> plan =
+      resident_pack(ls, (unsigned)w.num_cu, [] { return resident_per_cu<R, LINK, 1, 2>(512); });
+  if (plan.empty()) return plan;
   // a device too full for a second set of slots keeps the launches per iteration
-  size_t fr = 0, tot = 0;
-  if (more && (hipMemGetInfo(&fr, &tot) != hipSuccess || more > fr / 2)) return {};
-  return resident_pack(ls, (unsigned)w.num_cu, [] { return resident_per_cu<R, LINK, 1, 2>(512); });
+  std::vector<size_t> need(cs.size());
+  size_t more = 0;
+  for (size_t l = 0; l < cs.size(); l++) {
+    need[l] = sizeof(Cx<R>) * (size_t)(3 * cs[l]->Vh * runs[l].nrhs) * std::min(runs[l].cap, runs[l].expect);
+    const size_t have = cs[l]->ws->cap[S_RES_H];
+    if (need[l] > have) more += need[l] - have;
+  }
+  if (more && more > device_free() / 2) return {};
+  for (size_t l = 0; l < cs.size(); l++)
+    if (!ws_try(*cs[l], S_RES_H, need[l])) return {};
+  for (BasisRun &br : runs) br.cap = std::min(br.cap, br.expect);
+  return plan;
 }
 
 static void resident_count(Context &c, const std::vector<ResidentLaunch> &plan) {
@@ -3039,7 +3044,7 @@ static int resident_launch(const std::vector<Context *> &cs, std::vector<BasisRu
     Context &c = *cs[rl.lat[q]];
     BasisRun &br = runs[rl.lat[q]];
     const long v = 3 * c.Vh;
-    Cx<R> *h = (Cx<R> *)ws_get(c, S_RES_H, resident_h_bytes<R>(c, br));
+    Cx<R> *h = (Cx<R> *)ws_get(c, S_RES_H, sizeof(Cx<R>) * (size_t)(v * br.nrhs) * br.cap);
     const int per = kResRing * kResCopies * res_copy(rl.nwg[q]), np = per * br.nrhs;
     unsigned long long *part = (unsigned long long *)ws_get(c, S_RES_PART, sizeof(unsigned long long) * np + 64);
     if (!h || !part) return -1;

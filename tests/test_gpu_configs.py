@@ -948,6 +948,48 @@ def test_power_iterations_in_one_launch(dims, monkeypatch):
     g.close()
 
 
+def test_one_launch_solve_takes_the_memory_its_iterations_need(monkeypatch):
+    """The second set of slots of a one-launch solve: after a correction of 24
+    systems has grown the handle's basis to 2.4 GB, solves of one system of
+    16^4 take slots for at most twice their iterations (128 at least; 64 MB for
+    the rest), and where those would be more than half of the free memory the
+    launches per iteration.  Solutions agree with those of a fresh handle
+    to 1e-9 (true residuals of 1e-10 |b|)."""
+    import torch
+    dims, mass = (16, 16, 16, 16), 0.05
+    lat = fields.Lattice(*dims)
+    U = fields.random_links(lat, 43, 0.3)
+    phi = fields.gauss_spinor(lat, 44, 1)
+    many, one = np.geomspace(1e-4, 2.0, 24), np.array([1e-3])
+    vector = 48 * lat.Vh
+    fresh = Gpu(dims, mass=mass, max_order=24)
+    fresh.init0(U)
+    fresh.init1(phi=phi)
+    fresh.multishift(one, 1e-10, relative=True, precision=0)
+    want = fresh.get_fermions("smf")
+    fresh.close()
+    g = Gpu(dims, mass=mass, max_order=24)
+    g.init0(U)
+    g.init1(phi=phi)
+    g.multishift(many, 1e-10, relative=True, precision=1)
+    say("basis grown")
+    free = torch.cuda.mem_get_info()[0]
+    monkeypatch.setenv("RHMC_FREE_BYTES", "1000000")
+    before = g.path_counters()["one_launch"]
+    g.multishift(one, 1e-10, relative=True, precision=0)
+    assert g.path_counters()["one_launch"] == before
+    assert rel(g.get_fermions("smf"), want) < 1e-9
+    monkeypatch.delenv("RHMC_FREE_BYTES")
+    for _ in range(4):
+        it = g.multishift(one, 1e-10, relative=True, precision=0)
+    assert g.path_counters()["one_launch"] > before
+    assert rel(g.get_fermions("smf"), want) < 1e-9
+    took = free - torch.cuda.mem_get_info()[0]
+    say("iterations", it, "memory", took)
+    assert took < max(128, 2 * it) * vector + (64 << 20)
+    g.close()
+
+
 @pytest.mark.parametrize("dims", [(4, 4, 4, 4), (16, 16, 16, 16), (24, 24, 24, 8)])
 def test_power_iterations_without_room_for_their_slots(dims, monkeypatch):
     """Where the 129 vectors of the many-per-launch form would take more than
