@@ -106,7 +106,7 @@ int gpu_create(const rhmc_gpu_params *p, rhmc_gpu_t *out) {
   Context &c = h->c;
   c.device = p->device;
   if (!hip_ok(c, hipSetDevice(p->device), "hipSetDevice")) { delete h; return RHMC_EHIP; }
-  host_stage_retain();
+  host_stage_retain(c.device);
   fill_dims(c, p->nx, p->ny, p->nz, p->nt, p->antiperiodic_t);
   c.mass = p->mass;
   c.beta = p->beta;
@@ -155,7 +155,7 @@ int gpu_destroy(rhmc_gpu_t h) {
   kernel_timing_release(c);
   workspace_destroy(c.ws);
   if (c.stream) hipStreamDestroy(c.stream);
-  host_stage_release();
+  host_stage_release(c.device);
   delete h;
   return RHMC_OK;
 }

@@ -238,9 +238,9 @@ void *scratch_get(Context &c, int use, size_t bytes);
 bool h2d(Context &c, void *dst, const void *src, size_t bytes);
 bool d2h_sync(Context &c, void *dst, const void *src, size_t bytes);
 
-// the pinned buffers of large host transfers (fields.hip): one use per context
-void host_stage_retain();
-void host_stage_release();
+// a device's pinned buffers for large host transfers (fields.hip): one use per context
+void host_stage_retain(int device);
+void host_stage_release(int device);
 
 // host helpers
 bool hip_ok(Context &c, hipError_t e, const char *what);

@@ -10,7 +10,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <vector>
 
@@ -1143,59 +1143,74 @@ int time_copy(Context &c, size_t bytes, int reps, double *ms) {
 // while the other is moved by the CPU): 4.4 ms and 4.0 ms; the bus alone
 // takes 2.8 ms, and more threads or larger chunks gain nothing.
 //
-// The pinned buffers (16 MB) serve every context of the process, one
-// transfer at a time, and are freed with the last context.  Allocating them
-// takes 3.5 ms, as long as they save on some 50 MB, so they are allocated by
-// the transfer that brings the large ones' total past kStageWorth.
+// The pinned buffers (16 MB) serve every context of a device, one transfer
+// at a time (the bus is theirs), and are freed with the last of them.
+// Allocating them takes 3.5 ms, as long as they save on some 50 MB, so they
+// are allocated by the transfer that brings the large ones' total past
+// kStageWorth.  Memory that the runtime knows (pinned or managed) takes its
+// own copy, which goes over the bus directly.
 constexpr int kStageThreads = 4;
 constexpr size_t kStageChunk = 2u << 20;
 constexpr size_t kStageMin = 8u << 20;  // smaller copies: the runtime's (two chunks a thread and more)
 constexpr size_t kStageWorth = 64u << 20;
 
 struct HostStage {
-  std::mutex m;
+  std::mutex m;  // buf and moved; held through a transfer
   char *buf = nullptr;
-  int users = 0;
   size_t moved = 0;  // bytes of the large transfers
+  std::atomic<int> users{0};
 };
-static HostStage &host_stage() {
-  static HostStage s;
-  return s;
+static HostStage &host_stage(int device) {
+  static HostStage s[64];
+  return s[device < 0 || device >= 64 ? 0 : device];
 }
-void host_stage_retain() {
-  HostStage &s = host_stage();
+void host_stage_retain(int device) { host_stage(device).users++; }
+void host_stage_release(int device) {
+  HostStage &s = host_stage(device);
+  if (--s.users) return;
   std::lock_guard<std::mutex> l(s.m);
-  s.users++;
+  if (s.users) return;  // a context made meanwhile
+  if (s.buf) hipHostFree(s.buf);
+  s.buf = nullptr;
+  s.moved = 0;
 }
-void host_stage_release() {
-  HostStage &s = host_stage();
-  std::lock_guard<std::mutex> l(s.m);
-  if (--s.users == 0) {
-    if (s.buf) hipHostFree(s.buf);
-    s.buf = nullptr;
-    s.moved = 0;
+
+static bool known_to_runtime(const void *p) {
+  hipPointerAttribute_t a = {};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
   }
+  return a.type != hipMemoryTypeUnregistered;
+}
+
+// whether a copy goes through the pinned buffers, which are there then (the
+// context, a user of them, keeps them)
+static bool host_staged(HostStage &s, const void *host, size_t bytes) {
+  if (bytes < kStageMin || known_to_runtime(host)) return false;
+  std::lock_guard<std::mutex> l(s.m);
+  if (s.moved <= kStageWorth) s.moved += bytes;
+  if (!s.buf && s.moved > kStageWorth &&
+      hipHostMalloc((void **)&s.buf, 2 * kStageThreads * kStageChunk, hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();
+    s.buf = nullptr;
+  }
+  return s.buf != nullptr;
 }
 
 // dev -> host (down) or host -> dev on c.stream; every caller synchronises
 // the stream before it returns to the user
 static bool host_copy(Context &c, void *dev, void *host, size_t bytes, bool down) {
-  HostStage &s = host_stage();
-  std::unique_lock<std::mutex> l(s.m, std::defer_lock);
-  if (bytes >= kStageMin) {
-    l.lock();
-    if (s.moved <= kStageWorth) s.moved += bytes;
-    if (!s.buf && s.moved > kStageWorth &&
-        hipHostMalloc((void **)&s.buf, 2 * kStageThreads * kStageChunk, hipHostMallocPortable) != hipSuccess) {
-      (void)hipGetLastError();
-      s.buf = nullptr;
-    }
-  }
-  if (bytes < kStageMin || !s.buf) {
+  HostStage &s = host_stage(c.device);
+  if (!host_staged(s, host, bytes)) {
     const hipError_t e = down ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, c.stream)
                               : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, c.stream);
     return hip_ok(c, e, "host transfer");
   }
+  // the stream's earlier work is over before the buffers are taken: others
+  // wait for a transfer, not for what it follows
+  if (!hip_ok(c, hipStreamSynchronize(c.stream), "host transfer")) return false;
+  std::lock_guard<std::mutex> l(s.m);
   c.path[RHMC_COUNT_STAGED]++;
   const size_t n = (bytes + kStageChunk - 1) / kStageChunk;
   std::atomic<size_t> next{0};
@@ -1248,7 +1263,7 @@ static bool host_copy(Context &c, void *dev, void *host, size_t bytes, bool down
   std::thread th[kStageThreads - 1];
   try {
     for (int k = 1; k < kStageThreads; k++) th[k - 1] = std::thread(worker, k);
-  } catch (const std::system_error &) {
+  } catch (const std::exception &) {
   }
   worker(0);
   for (std::thread &t : th)

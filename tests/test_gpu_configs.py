@@ -1111,6 +1111,33 @@ def test_host_transfers_round_trip(dims):
     assert not err, err
 
 
+def test_host_transfers_of_pinned_arrays():
+    """Links of 75 MB from and to ordinary arrays go through the pinned chunks,
+    from and to arrays that are pinned already directly; both come back bit
+    for bit."""
+    import ctypes as C
+
+    import torch
+    dims = (32, 32, 16, 8)
+    lat = fields.Lattice(*dims)
+    U = fields.random_links(lat, 75, 0.3)
+    say("pinned transfers", dims)
+    pin = torch.empty(U.size * 2, dtype=torch.float64, pin_memory=True).numpy()
+    pin[:] = U.view(np.float64).ravel()
+    g = Gpu(dims, mass=0.1)
+    g.init0(U)
+    staged = g.path_counters()["staged"]
+    assert staged >= 1
+    assert g.L.gpu_init0(g.h, pin.ctypes.data_as(C.c_void_p)) == 0
+    pin[:] = 0.0
+    assert g.L.gpu_end(g.h, pin.ctypes.data_as(C.c_void_p), None, None) == 0
+    assert g.path_counters()["staged"] == staged
+    assert np.array_equal(pin, U.view(np.float64).ravel())
+    assert np.array_equal(g.end(ipdot=False, momenta=False)[0], U)
+    assert g.path_counters()["staged"] == staged + 1
+    g.close()
+
+
 # ------------------------------------------------------------- gauge force
 @pytest.mark.parametrize("dims,antiperiodic", [((2, 2, 2, 2), True), ((2, 4, 6, 8), True), ((8, 2, 4, 2), False),
                                                ((6, 6, 6, 6), True), ((16, 16, 16, 8), True), ((10, 8, 6, 4), False)])
