@@ -567,8 +567,9 @@ __global__ __launch_bounds__(64 * kResMaxWaves) __attribute__((amdgpu_waves_per_
 // iteration i is in slot (base + i) mod (n + 1) of r.basis, h in slot i of
 // r.h, so no slot is read before it is written in a launch.  norms[0] is
 // |p|^2 at the start, norms[i] that of iteration i, norms[n+1] the
-// iterations run (-1: the grid gave up); the launch ends at the first one
-// whose norm changed by at most tol relatively.
+// iterations run (-1: the grid gave up), norms[n+2] whether the last met the
+// test; the launch ends at the first one whose norm changed by at most tol
+// relatively.
 struct PowArgs {
   ResArgs r;
   double pa, pb, tol;
@@ -613,7 +614,8 @@ __global__ __launch_bounds__(64 * kResMaxWaves) __attribute__((amdgpu_waves_per_
   __syncthreads();
   double n2 = q.norms[0], prev = sqrt(n2);
   int i = 0;
-  for (bool met = false; i < q.n && !met; i++) {
+  bool met = false;
+  for (; i < q.n && !met; i++) {
     const C *in = ring + (long)((q.base + i) % (q.n + 1)) * a.stride;
     C *out = ring + (long)((q.base + i + 1) % (q.n + 1)) * a.stride, *hs = (C *)a.h + (long)i * a.stride;
     double v[1] = {0.0};
@@ -649,7 +651,10 @@ __global__ __launch_bounds__(64 * kResMaxWaves) __attribute__((amdgpu_waves_per_
     met = !(fabs(prev - norm) / norm > q.tol);
     prev = norm;
   }
-  if (wg == 0 && threadIdx.x == 0) q.norms[q.n + 1] = s.aborted ? -1.0 : (double)i;
+  if (wg == 0 && threadIdx.x == 0) {
+    q.norms[q.n + 1] = s.aborted ? -1.0 : (double)i;
+    q.norms[q.n + 2] = met ? 1.0 : 0.0;
+  }
 }
 
 }  // namespace rhmc

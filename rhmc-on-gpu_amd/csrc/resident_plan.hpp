@@ -1,5 +1,6 @@
 // resident_plan.hpp -- how the systems of a one-launch solve (resident.hpp) are
-// laid over a device's workgroups.  Host code without a device call.
+// laid over a device's workgroups, and where its power iterations stop.  Host
+// code without a device call.
 #pragma once
 
 #include <algorithm>
@@ -124,6 +125,16 @@ std::vector<ResidentLaunch> resident_pack(const std::vector<ResidentLattice> &ls
     out[q].total += t;
   }
   return out.size() <= 3 ? out : std::vector<ResidentLaunch>();
+}
+
+// The result of a launch of power iterations i0, i0+1, ...: it ran `ran` of
+// them, the last of which met the test or not.  The kernel is the judge (what
+// it did not run was not written); the host adds the largest number of
+// iterations.  Returns the iteration that gives the result, 0 to go on; q:
+// its place in the launch, from 1.
+inline int power_stop(int i0, int ran, bool met, int most, int &q) {
+  q = std::min(ran, most - i0 + 1);
+  return met || i0 + ran > most ? i0 + q - 1 : 0;
 }
 
 }  // namespace rhmc

@@ -4007,7 +4007,7 @@ static int power_resident(Context &c, const double2 *start, double tol, double p
   // 129 vectors, at most 400 MB, where the launches take three
   double2 *p = (double2 *)ws_try(c, S_PW1, sizeof(double2) * n * (2 * kPowSmall + 1));
   if (!p) return 1;
-  double *pn = (double *)ws_get(c, S_PWN, sizeof(double) * (kPowSmall + 2));
+  double *pn = (double *)ws_get(c, S_PWN, sizeof(double) * (kPowSmall + 3));
   const int np = kResRing * kResCopies * res_copy(nwg);
   unsigned long long *part = (unsigned long long *)ws_get(c, S_RES_PART, sizeof(unsigned long long) * np + 64);
   if (!pn || !part) return -1;
@@ -4029,13 +4029,13 @@ static int power_resident(Context &c, const double2 *start, double tol, double p
   a.wait = wait ? atoll(wait) : kResWaitTicks;
   c.path[RHMC_COUNT_POWER]++;
   ResidentShare share(c.device, (double)total / w->num_cu);
-  double h[kPowSmall + 2];
+  double h[kPowSmall + 3];
   for (int i0 = 1;; i0 += kPowSmall) {
     hipLaunchKernelGGL(k_res_init, dim3(std::min(256, (np + kBlock - 1) / kBlock)), dim3(kBlock), 0, c.stream, part,
                        np, a.r.abort);
     if (sites == 1) hipLaunchKernelGGL(k_pow_resident<1>, dim3(total), dim3(threads), 0, c.stream, a);
     else hipLaunchKernelGGL(k_pow_resident<2>, dim3(total), dim3(threads), 0, c.stream, a);
-    if (!hip_ok(c, hipGetLastError(), "power iterations") || !d2h_sync(c, h, pn, sizeof(double) * (kPowSmall + 2)))
+    if (!hip_ok(c, hipGetLastError(), "power iterations") || !d2h_sync(c, h, pn, sizeof(h)))
       return -1;
     const int ran = (int)h[kPowSmall + 1];
     if (ran < 0) {
@@ -4043,7 +4043,11 @@ static int power_resident(Context &c, const double2 *start, double tol, double p
       w->resident_off = true;
       return 1;
     }
-    if ((*loops = power_met(h, i0, ran, tol, *norm))) return 0;
+    int q = 0;
+    if ((*loops = power_stop(i0, ran, h[kPowSmall + 2] != 0.0, kPowMax, q))) {
+      *norm = sqrt(h[q]);
+      return 0;
+    }
     // the last vector, in its slot of the ring, is the next launch's first
     a.base = (a.base + kPowSmall) % (kPowSmall + 1);
     hipMemcpyAsync(pn, pn + kPowSmall, sizeof(double), hipMemcpyDeviceToDevice, c.stream);

@@ -25,6 +25,8 @@ extern "C" int plan(int n, const long *vh, const int *nrhs, int whole, int cus, 
   }
   return (int)(o - out);
 }
+// the iteration that gives the result (0: go on); its place in the launch to *q
+extern "C" int stop(int i0, int ran, int met, int most, int *q) { return power_stop(i0, ran, met != 0, most, *q); }
 extern "C" int max_members() { return kResMaxMembers; }
 """
 
@@ -102,3 +104,18 @@ def test_plan_of_many_small_systems(lib):
     small, big = 8 ** 3 * 4 // 2, 16 ** 4 // 2
     for lats in ([(small, 8)] * 12, [(small, 5)] * 12, [(small, 5)] * 16, [(big, 1)] + [(small, 8)] * 3):
         check(lib, lats, True, 256, 2)
+
+
+# (first iteration, iterations run, met) of launches of 64, at most 20000: (iteration of the result or 0, its place)
+@pytest.mark.parametrize("i0,ran,met,result,place", [
+    (1, 1, 1, 1, 1), (1, 10, 1, 10, 10), (1, 64, 1, 64, 64), (1, 64, 0, 0, None), (65, 3, 1, 67, 3),
+    (19905, 64, 0, 0, None), (19969, 64, 0, 20000, 32), (19969, 32, 1, 20000, 32), (19969, 31, 1, 19999, 31),
+    (19969, 33, 1, 20000, 32), (19969, 64, 1, 20000, 32)])
+def test_power_iterations_stop_where_the_kernel_did(lib, i0, ran, met, result, place):
+    """A launch that ended early is the end whatever the host would make of
+    the norms (what it did not run holds nothing); the iterations past the
+    largest number are not used."""
+    q = C.c_int()
+    assert lib.stop(i0, ran, met, 20000, C.byref(q)) == result
+    if result:
+        assert q.value == place
