@@ -43,7 +43,10 @@ constexpr int kResAborted = 2;            // MsState::nonfinite of system 0: the
 constexpr int kResRing = 4;               // reduction slots in use in turn
 constexpr int kResCopies = 8;             // copies of the slots, one per XCD
 constexpr unsigned long long kResNone = ~0ull;  // a partial that has not arrived
-constexpr long long kResWaitTicks = 400000000ll;  // bound of a wait: 4 s of the 100 MHz wall clock
+// Bound of a wait: 50 ms of the 100 MHz wall clock.  A meeting takes 1.4-3 us
+// and a whole solve a few milliseconds: a workgroup that has not come by then
+// has no place on the device.
+constexpr long long kResWaitTicks = 5000000ll;
 constexpr int kResMaxWaves = 8;           // waves of a workgroup (512 lanes)
 
 // one member of a launch: nvec right-hand sides of one lattice's solve

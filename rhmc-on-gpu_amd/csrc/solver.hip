@@ -81,7 +81,7 @@ struct Workspace {
   std::map<unsigned long long, int> group_tuned;  // lockstep launch shape per group composition
   long basis_kmax[3] = {0, 0, 0};              // most basis iterations a FP32 / FP64 solve, a correction needed
   int num_cu = 0;                              // compute units of the device
-  bool resident_off = false;                   // a one-launch solve gave up waiting (device shared): not used again
+  int resident_rest = 0;                       // one-launch work left to the launches since some gave up waiting
   void *buf[S_COUNT] = {};
   size_t cap[S_COUNT] = {};
   unsigned *counter = nullptr;
@@ -2988,6 +2988,21 @@ static int resident_per_cu(int threads) {
   }
   return n;
 }
+// After one-launch work has given up, which means that another process holds
+// part of the device, the next kResidentRest solves and bounds of the handle
+// use the launches per iteration at once: a wait in vain (50 ms) is then 0.2
+// ms for each of them, and the handle finds out when the device is free.
+constexpr int kResidentRest = 256;
+static void resident_gave_up(Context &c) {
+  c.path[RHMC_COUNT_GAVE_UP]++;
+  c.ws->resident_rest = kResidentRest;
+}
+static bool resident_resting(Workspace &w) {
+  if (w.resident_rest == 0) return false;
+  w.resident_rest--;
+  return true;
+}
+
 // The launches of a solve over one or several lattices (resident_pack); empty
 // where the launches per iteration are used.  A run that is placed has its
 // slots bounded by those its iterations so far ask for (the basis allocation
@@ -2995,8 +3010,8 @@ static int resident_per_cu(int threads) {
 // and the h slots allocated; one that fills them is continued.
 template <typename R, int LINK>
 static std::vector<ResidentLaunch> resident_plan(const std::vector<Context *> &cs, std::vector<BasisRun> &runs) {
-  const Workspace &w = *cs[0]->ws;
-  if (w.resident_off || w.num_cu < 8 || getenv("RHMC_DSLASH_NR")) return {};
+  Workspace &w = *cs[0]->ws;
+  if (w.num_cu < 8 || getenv("RHMC_DSLASH_NR")) return {};
   std::vector<ResidentLattice> ls;
   for (size_t l = 0; l < cs.size(); l++) {
     const size_t vb = (size_t)3 * cs[l]->Vh * sizeof(Cx<R>);
@@ -3006,7 +3021,7 @@ static std::vector<ResidentLaunch> resident_plan(const std::vector<Context *> &c
   }
   std::vector<ResidentLaunch> plan =
       resident_pack(ls, (unsigned)w.num_cu, [] { return resident_per_cu<R, LINK, 1, 2>(512); });
-  if (plan.empty()) return plan;
+  if (plan.empty() || resident_resting(w)) return {};
   // a device too full for a second set of slots keeps the launches per iteration
   std::vector<size_t> need(cs.size());
   size_t more = 0;
@@ -3108,8 +3123,7 @@ static int ms_cg_basis(Context &c, const double2 *b, int nrhs, int nshift, const
       if (rc < 0) hipStreamSynchronize(c.stream);  // nothing of it in flight when the share is given back
     }
     if (rc != kResidentGaveUp) return rc;
-    c.path[RHMC_COUNT_GAVE_UP]++;
-    c.ws->resident_off = true;
+    resident_gave_up(c);
     br = BasisRun();
     rc = bms_setup<R, LINK>(c, br, b, nrhs, nshift, shifts, res_abs, max_iter, iterc, tol_abs, tol_rel, sys);
     if (rc) return rc;
@@ -3312,8 +3326,7 @@ static int ms_cg_basis_group(std::vector<Context *> &cs, std::vector<GroupJob> &
       if (rc) hipStreamSynchronize(c0.stream);
     }
     if (rc != kResidentGaveUp) return rc;
-    c0.path[RHMC_COUNT_GAVE_UP]++;
-    c0.ws->resident_off = true;
+    resident_gave_up(c0);
     if ((rc = setup())) return rc;
   }
   // the shape candidates run iteration 1 and read the iteration counter: on a
@@ -3997,12 +4010,12 @@ static int power_met(const double *h, int i0, int n, double tol, double &norm) {
 static int power_resident(Context &c, const double2 *start, double tol, double pa, double pb, double *norm,
                           int *loops) {
   Workspace *w = c.ws;
-  if (w->resident_off || w->num_cu < 8 || getenv("RHMC_DSLASH_NR")) return 1;
+  if (w->num_cu < 8 || getenv("RHMC_DSLASH_NR")) return 1;
   int threads = 256, sites = 1, nwg = 0;
   unsigned total = resident_wgs(c.Vh, threads, sites, nwg);
   if (total > (unsigned)w->num_cu) total = resident_wgs(c.Vh, threads = 512, sites, nwg);
   if (total > (unsigned)w->num_cu) total = resident_wgs(c.Vh, threads, sites = 2, nwg);
-  if (total > (unsigned)w->num_cu) return 1;
+  if (total > (unsigned)w->num_cu || resident_resting(*w)) return 1;
   const long n = 3 * c.Vh;  // whole cache lines: V/2 is a multiple of 8
   // 129 vectors, at most 400 MB, where the launches take three
   double2 *p = (double2 *)ws_try(c, S_PW1, sizeof(double2) * n * (2 * kPowSmall + 1));
@@ -4039,8 +4052,7 @@ static int power_resident(Context &c, const double2 *start, double tol, double p
       return -1;
     const int ran = (int)h[kPowSmall + 1];
     if (ran < 0) {
-      c.path[RHMC_COUNT_GAVE_UP]++;
-      w->resident_off = true;
+      resident_gave_up(c);
       return 1;
     }
     int q = 0;

@@ -948,6 +948,33 @@ def test_power_iterations_in_one_launch(dims, monkeypatch):
     g.close()
 
 
+def test_one_launch_solves_are_tried_again(monkeypatch):
+    """After a solve that gave up, 256 solves use the launches per iteration;
+    then one launch is tried again, and used from there on when it is let."""
+    dims = (8, 8, 8, 4)
+    lat = fields.Lattice(*dims)
+    g = Gpu(dims, mass=0.5, max_order=1)
+    g.init0(fields.random_links(lat, 45, 0.3))
+    g.init1(phi=fields.gauss_spinor(lat, 46, 1))
+
+    def solves(n):
+        for _ in range(n):
+            g.multishift([1.0], 1e-1, relative=True, precision=0)
+        c = g.path_counters()
+        return c["one_launch"], c["gave_up"]
+
+    monkeypatch.setenv("RHMC_RESIDENT_WAIT", "0")
+    say("gives up, rests")
+    assert solves(1) == (1, 1)
+    assert solves(256) == (1, 1)
+    assert solves(1) == (2, 2)
+    monkeypatch.delenv("RHMC_RESIDENT_WAIT")
+    say("rests, then runs")
+    assert solves(256) == (2, 2)
+    assert solves(3) == (5, 2)
+    g.close()
+
+
 def test_one_launch_solve_takes_the_memory_its_iterations_need(monkeypatch):
     """The second set of slots of a one-launch solve: after a correction of 24
     systems has grown the handle's basis to 2.4 GB, solves of one system of
