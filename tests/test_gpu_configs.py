@@ -948,6 +948,53 @@ def test_power_iterations_in_one_launch(dims, monkeypatch):
     g.close()
 
 
+def test_one_launch_solves_of_several_threads():
+    """Four handles, each in a thread of its own: two of 16^4, whose one-launch
+    solves fill the device's workgroups one handle at a time, and two small
+    ones, whose solves run beside each other.  Solutions and bounds are those
+    of the handle working alone, bit for bit (every sum has a fixed order), and
+    no solve gives up."""
+    import threading
+    mass, b = 0.05, np.geomspace(1e-4, 2.0, 7)
+    handles = []
+    for i, dims in enumerate([(16, 16, 16, 16), (8, 8, 8, 4), (16, 16, 16, 16), (6, 4, 4, 6)]):
+        lat = fields.Lattice(*dims)
+        g = Gpu(dims, mass=mass, n_pf=2, max_order=7)
+        g.init0(fields.random_links(lat, 47 + i, 0.3))
+        g.init1(phi=fields.gauss_spinor(lat, 57 + i, 2))
+        handles.append(g)
+
+    def work(g):
+        g.multishift(b, 1e-10, relative=True, precision=0)
+        x = g.get_fermions("smf")
+        return x, g.find_max(1e-4, seed=9)
+
+    say("threads")
+    # the slots follow the iterations: settled after a few solves
+    alone = [[work(g) for _ in range(4)][-1] for g in handles]
+    ran = [g.path_counters()["one_launch"] for g in handles]
+    err = []
+
+    def thread(g, want):
+        try:
+            for _ in range(10):
+                x, mx = work(g)
+                assert np.array_equal(x, want[0]) and mx == want[1]
+        except BaseException as e:  # reported by the main thread
+            err.append(e)
+
+    th = [threading.Thread(target=thread, args=a) for a in zip(handles, alone)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not err, err
+    for g, n in zip(handles, ran):
+        c = g.path_counters()
+        assert c["one_launch"] >= n + 10 and c["power"] == 14 and c["gave_up"] == 0
+        g.close()
+
+
 def test_one_launch_solves_are_tried_again(monkeypatch):
     """After a solve that gave up, 256 solves use the launches per iteration;
     then one launch is tried again, and used from there on when it is let."""
