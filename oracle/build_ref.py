@@ -8,7 +8,7 @@
    each configuration is placed first on the include path).
 
 Outputs go only into oracle/_ref/ (git-ignored).  Step 2 is skipped when
-/root/reference is absent (e.g. on a machine without the reference).
+/root/reference does not hold the sources (e.g. on a machine without them).
 """
 from __future__ import annotations
 
@@ -46,6 +46,12 @@ REF_SOURCES = [
     "lib/Measurements/gaugemeas.cc",
     "lib/Measurements/chiralmeas.cc",
 ]
+
+
+def have_reference() -> bool:
+    """Whether the reference's sources are there (its directory may be empty)."""
+    return os.path.isfile(os.path.join(REF, REF_SOURCES[0]))
+
 
 # Compile-time configurations for the golden vectors.  Keys are the constant
 # names the reference reads from include/parameters.h.
@@ -123,7 +129,7 @@ def build_oracle_lib():
 
 
 def build_ref(name: str, force: bool = False):
-    if not os.path.isdir(REF):
+    if not have_reference():
         return None
     cfg = CONFIGS[name]
     bdir = os.path.join(OUT, name)

@@ -7,7 +7,7 @@ together with compat/reference_shim.cc (the lib/Cuda entry points on the C
 ABI) and the golden-vector harness oracle/ref_harness.cc.  The result,
 oracle/_ref/<cfg>_gpu/ref_harness_gpu, runs the reference's own update()
 with every device call served by this library.  Output stays in oracle/_ref/
-(git-ignored).  Skipped when /root/reference is absent.
+(git-ignored).  Skipped when /root/reference does not hold the sources.
 """
 from __future__ import annotations
 
@@ -38,7 +38,7 @@ GPU_SOURCES = br.REF_SOURCES + [
 
 
 def build(name: str, force: bool = False):
-    if not os.path.isdir(br.REF):
+    if not br.have_reference():
         return None
     lib = os.path.join(PKG, "rhmc_amd", "librhmc_amd.so")
     if not os.path.exists(lib):

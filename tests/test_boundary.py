@@ -92,3 +92,19 @@ def test_every_wrapper_converts_its_arguments():
             pass
         except (TypeError, C.ArgumentError) as e:
             raise AssertionError(f"call {k}: {e}")
+
+
+def test_reference_builds_need_its_sources(tmp_path, monkeypatch):
+    """Without the reference's sources, also where its directory is there but
+    empty, both builds that compile them do nothing."""
+    import importlib.util
+    path = os.path.join(os.path.dirname(__file__), "..", "rhmc-on-gpu_amd", "compat", "build_compat.py")
+    spec = importlib.util.spec_from_file_location("build_compat", path)
+    bc = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bc)
+    monkeypatch.setattr(bc.br, "OUT", str(tmp_path / "out"))
+    for ref in (tmp_path, tmp_path / "absent"):
+        monkeypatch.setattr(bc.br, "REF", str(ref))
+        assert bc.br.build_ref("t4", force=True) is None
+        assert bc.build("t4", force=True) is None
+    assert not os.path.exists(bc.br.OUT)
