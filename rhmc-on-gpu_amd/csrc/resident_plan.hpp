@@ -1,9 +1,11 @@
 // resident_plan.hpp -- how the systems of a one-launch solve (resident.hpp) are
-// laid over a device's workgroups, and where its power iterations stop.  Host
-// code without a device call.
+// laid over a device's workgroups, where its power iterations stop, and the
+// share of the device that each takes.  Host code without a device call.
 #pragma once
 
 #include <algorithm>
+#include <condition_variable>
+#include <mutex>
 #include <vector>
 
 namespace rhmc {
@@ -136,5 +138,50 @@ inline int power_stop(int i0, int ran, bool met, int most, int &q) {
   q = std::min(ran, most - i0 + 1);
   return met || i0 + ran > most ? i0 + q - 1 : 0;
 }
+
+// Workgroups of the one-launch solves in flight on a device, as a share of
+// its compute units: solves of several handles (threads) run at the same
+// time only while all their workgroups fit, at most one per CU, so that
+// every grid is resident as a whole.  Shares are given in the order in which
+// they were asked for: one of the whole device would else wait for as long as
+// smaller ones overlap.
+class ResidentShare {
+ public:
+  ResidentShare(int device, double share) : d_(device < 0 || device >= kDevices ? 0 : device), s_(share) {
+    Slots &t = slots();
+    std::unique_lock<std::mutex> l(t.m);
+    const unsigned long turn = t.asked[d_]++;
+    t.cv.wait(l, [&] { return t.given[d_] == turn && t.used[d_] + s_ <= 1.0 + 1e-9; });
+    t.used[d_] += s_;
+    t.given[d_]++;
+    l.unlock();
+    t.cv.notify_all();  // the next in turn may fit beside it
+  }
+  ~ResidentShare() {
+    Slots &t = slots();
+    {
+      std::lock_guard<std::mutex> l(t.m);
+      t.used[d_] -= s_;
+    }
+    t.cv.notify_all();
+  }
+  ResidentShare(const ResidentShare &) = delete;
+  ResidentShare &operator=(const ResidentShare &) = delete;
+
+ private:
+  static constexpr int kDevices = 64;
+  struct Slots {
+    std::mutex m;
+    std::condition_variable cv;
+    double used[kDevices] = {};
+    unsigned long asked[kDevices] = {}, given[kDevices] = {};
+  };
+  static Slots &slots() {
+    static Slots t;
+    return t;
+  }
+  int d_;
+  double s_;
+};
 
 }  // namespace rhmc

@@ -25,12 +25,10 @@
 
 #include <algorithm>
 #include <cmath>
-#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
-#include <mutex>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -2940,44 +2938,6 @@ static int bms_finish(Context &c, BasisRun &br, double2 *x, int *iters_out, floa
     }
   return 0;
 }
-
-// Workgroups of the one-launch solves in flight on a device, as a share of
-// its compute units: solves of several handles (threads) run at the same
-// time only while all their workgroups fit, at most one per CU, so that
-// every grid is resident as a whole.
-class ResidentShare {
- public:
-  ResidentShare(int device, double share) : d_(device < 0 || device >= kDevices ? 0 : device), s_(share) {
-    Slots &t = slots();
-    std::unique_lock<std::mutex> l(t.m);
-    t.cv.wait(l, [&] { return t.used[d_] + s_ <= 1.0 + 1e-9; });
-    t.used[d_] += s_;
-  }
-  ~ResidentShare() {
-    Slots &t = slots();
-    {
-      std::lock_guard<std::mutex> l(t.m);
-      t.used[d_] -= s_;
-    }
-    t.cv.notify_all();
-  }
-  ResidentShare(const ResidentShare &) = delete;
-  ResidentShare &operator=(const ResidentShare &) = delete;
-
- private:
-  static constexpr int kDevices = 64;
-  struct Slots {
-    std::mutex m;
-    std::condition_variable cv;
-    double used[kDevices] = {};
-  };
-  static Slots &slots() {
-    static Slots t;
-    return t;
-  }
-  int d_;
-  double s_;
-};
 
 template <typename R, int LINK, int NR, int P>
 static int resident_per_cu(int threads) {

@@ -11,7 +11,32 @@ ROOT = os.path.abspath(os.path.join(os.path.dirname(__file__), ".."))
 
 SHIM = r"""
 #include "resident_plan.hpp"
+#include <atomic>
+#include <chrono>
+#include <thread>
 using namespace rhmc;
+// two threads that take a tenth each over and over, never both without it for
+// long: how often they did before a third got the whole, at most limit
+extern "C" int turns(int limit) {
+  std::atomic<int> n{0};
+  std::atomic<bool> waiting{false}, got{false};
+  auto small = [&](int ms) {
+    while (!got && n < limit) {
+      ResidentShare s(0, 0.1);
+      if (waiting) n++;
+      std::this_thread::sleep_for(std::chrono::milliseconds(ms));
+    }
+  };
+  std::thread a(small, 3), b(small, 4);
+  std::this_thread::sleep_for(std::chrono::milliseconds(20));
+  std::thread c([&] {
+    waiting = true;
+    ResidentShare s(0, 1.0);
+    got = true;
+  });
+  a.join(); b.join(); c.join();
+  return n;
+}
 // out: launches, then of each nr, threads, members, total, lattices, and of each lattice index, sites, nwg
 extern "C" int plan(int n, const long *vh, const int *nrhs, int whole, int cus, int per_cu, int *out) {
   std::vector<ResidentLattice> ls;
@@ -36,7 +61,7 @@ def lib(tmp_path_factory):
     d = tmp_path_factory.mktemp("plan")
     src, so = d / "shim.cpp", d / "shim.so"
     src.write_text(SHIM)
-    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I",
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-pthread", "-shared", "-fPIC", "-I",
                     os.path.join(ROOT, "rhmc-on-gpu_amd", "csrc"), str(src), "-o", str(so)], check=True)
     return C.CDLL(str(so))
 
@@ -119,3 +144,10 @@ def test_power_iterations_stop_where_the_kernel_did(lib, i0, ran, met, result, p
     assert lib.stop(i0, ran, met, 20000, C.byref(q)) == result
     if result:
         assert q.value == place
+
+
+def test_whole_device_gets_its_turn(lib):
+    """A solve that needs every compute unit comes before those that ask for
+    theirs after it: at most the share that each of two other threads was about
+    to take when it began to wait."""
+    assert lib.turns(200) <= 4
