@@ -93,7 +93,8 @@ def dslash_traffic(table, Vh, nrhs, mode=0, red=0):
 
 
 KERNEL_SOURCES = ("rhmc-on-gpu_amd/csrc/solver.hip", "rhmc-on-gpu_amd/csrc/lattice.hpp",
-                  "rhmc-on-gpu_amd/csrc/context.hpp")
+                  "rhmc-on-gpu_amd/csrc/context.hpp", "rhmc-on-gpu_amd/csrc/resident.hpp",
+                  "rhmc-on-gpu_amd/csrc/resident_plan.hpp")
 
 
 def kernel_source_hash():
@@ -108,8 +109,9 @@ def kernel_source_hash():
 
 
 def counters_from(fetch_dir, write_dir, out_path):
-    """profiles/dslash_32c8_counters.json from two rocprofv3 --pmc runs of
-    `bench.py --dslash-only` (FETCH_SIZE, then WRITE_SIZE; csv output): per
+    """profiles/dslash_32c8_counters.json from rocprofv3 --pmc runs of
+    `bench.py --dslash-only` (FETCH_SIZE in one folder, WRITE_SIZE in the
+    other; csv output, of one run or of several with other launch shapes): per
     (kernel, grid) the mean counter per dispatch in KiB, scaled by the factor
     that makes the copy probe (1 GiB read + 1 GiB written) read its known
     size, with the SHA-256 of the kernel sources it was taken on.  Dispatches
@@ -126,8 +128,8 @@ def counters_from(fetch_dir, write_dir, out_path):
                     if row["Counter_Name"] != counter:
                         continue
                     k = (row["Kernel_Name"], int(row["Grid_Size"]))
-                    acc.setdefault(k, {})[row["Dispatch_Id"]] = acc.get(k, {}).get(row["Dispatch_Id"], 0.0) + \
-                        float(row["Counter_Value"])
+                    d = (f, row["Dispatch_Id"])
+                    acc.setdefault(k, {})[d] = acc.get(k, {}).get(d, 0.0) + float(row["Counter_Value"])
         out = {}
         for k, v in acc.items():
             # a solve's last chunk launches after every system has stopped exit

@@ -88,3 +88,35 @@ def test_bench_refuses_more_than_one_gpu():
                        text=True, timeout=120)
     assert p.returncode == 2
     assert "one GPU" in json.loads(p.stdout.strip().splitlines()[-1])["error"]
+
+
+def test_counters_of_several_runs(tmp_path):
+    """Runs with other launch shapes, in folders of their own below one: the
+    dispatches of two runs with the same numbers are different dispatches."""
+    gib_kib = float(1 << 20)
+    for run, grid in (("a", 131072), ("b", 262144)):
+        for counter, probe, v in (("FETCH_SIZE", 0.5, 60000.0), ("WRITE_SIZE", 1.0, 24000.0)):
+            write_run(str(tmp_path / counter / run), counter,
+                      [(PROBE, 2097152, [probe * gib_kib] * 3), (HOP, grid, [v])])
+    out = bench.counters_from(str(tmp_path / "FETCH_SIZE"), str(tmp_path / "WRITE_SIZE"), str(tmp_path / "c.json"))
+    assert abs(out["factors"]["fetch"] - 2.0) < 1e-12 and abs(out["factors"]["write"] - 1.0) < 1e-12
+    for grid in (131072, 262144):
+        k = out["kernels"][f"{HOP}|{grid}"]
+        assert k["dispatches"] == 1
+        assert abs(k["read_bytes"] - 60000.0 * 1024 * 2.0) < 1e-6 and abs(k["write_bytes"] - 24000.0 * 1024) < 1e-6
+
+
+def test_profile_hash_covers_the_solver_s_own_headers():
+    """Every header of the kernel folder that the solver's source includes,
+    directly or through another, is in the hash that guards a profile."""
+    import re
+    csrc = os.path.join(ROOT, "rhmc-on-gpu_amd", "csrc")
+    todo, seen = ["solver.hip"], set()
+    while todo:
+        f = todo.pop()
+        if f in seen or not os.path.exists(os.path.join(csrc, f)):
+            continue
+        seen.add(f)
+        with open(os.path.join(csrc, f)) as fh:
+            todo += re.findall(r'^\s*#include "([^"]+)"', fh.read(), re.M)
+    assert {"rhmc-on-gpu_amd/csrc/" + f for f in seen} == set(bench.KERNEL_SOURCES)
