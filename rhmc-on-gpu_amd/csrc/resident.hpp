@@ -541,7 +541,8 @@ struct ResGroup {
 static_assert(sizeof(ResGroup) <= 4000, "kernel arguments");
 
 // Waves per SIMD the kernel is compiled for: FP32 with one system, the form
-// that several lattices share, keeps two workgroups of 512 lanes per CU.
+// that several lattices share, keeps two workgroups of 512 lanes per CU (with
+// two sites per lane it spills 15 of its 128 registers).
 template <typename R, int NR>
 constexpr int res_waves() {
   return sizeof(R) == 4 && NR == 1 ? 4 : 2;
